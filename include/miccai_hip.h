@@ -359,7 +359,9 @@ int mh_cmf_solve_batched(mh_ctx *ctx, float *u_dev, int nsolves, const float *w_
  * one per thread). Results do not depend on the schedule, bit for bit. */
 int mh_cmf_batched_set_schedule(mh_ctx *ctx, int group, int visit);
 /* Multi-level sweep of mh_cmf_solve_batched's groups (no counterpart in the
- * reference). 0 (default): when the groups run one after another and the
+ * reference). 0 (default): solves that fit the device's registers stay on the
+ * chip (see mh_cmf_set_sweep; of three solves or more of 800,000 voxels or
+ * more the first two tune the sweeps, once per dims). Otherwise, when the groups run one after another and the
  * single-solve tuner picks a sweep for these dims (it is run on a probe copy
  * of solve 0 if it has not been for these dims), the solves run through a
  * sweep in pairs (two per thread) where the volume allows: the first group's
@@ -371,7 +373,11 @@ int mh_cmf_batched_set_schedule(mh_ctx *ctx, int group, int visit);
  * tuned one. Results do not depend on it, bit for bit. */
 int mh_cmf_batched_set_sweep(mh_ctx *ctx, int mode);
 /* Multi-level sweep of mh_cmf_solve on this context (no counterpart in the
- * reference): unsupervised constant-eigenvalue solves may advance two, three
+ * reference). In mode 0 (default) a solve whose volume fits the device's
+ * registers (about 2^21 voxels with constant eigenvalues (l0, l1, l1), half
+ * of that otherwise) stays on the chip from its first iteration to its last,
+ * unless another such solve is running on the device; what follows is for the
+ * others. Unsupervised constant-eigenvalue solves may advance two, three
  * or four iterations per pass over the state (temporal blocking along axis
  * 0; tile shapes 1-5 two levels, 6-7 three, 8-9 four). mode 0
  * (default) tunes: the second mh_cmf_solve of a volume shape on this context

@@ -1,0 +1,673 @@
+// Max-flow solves whose whole state stays on the chip.
+//
+// The state and inputs of a voxel are 12 to 19 floats; the 256 compute units
+// hold 128 MB of registers, so a volume of up to 2^21 voxels (128^3) fits. A
+// volume is cut into bricks of V planes x b1 x b2 voxels, one work-group per
+// brick and compute unit, a thread per in-plane position holding its V voxels
+// along axis 0 in registers for the whole solve: the fields are read once, u
+// is written once, and an iteration moves nothing through memory but the
+// brick faces.
+//
+// In-plane neighbours go through LDS, axis-0 neighbours are the thread's own
+// registers, and the faces of neighbouring bricks travel as tagged words: a
+// 64-bit store carries the iteration's tag beside the value, and the receiver
+// polls the word itself until the tag is the one it waits for, so that no flag,
+// fence or cache flush orders the exchange (one hop measures 1.0 us for 256
+// words, 1.3 us for 1024). One iteration is
+//   p-step, planes downwards: the top plane's h0, the last row's h1 and the
+//     last column's h2 go to the next bricks as they are formed;
+//   receive the previous bricks' h0, h1, h2; barrier;
+//   u-step, planes upwards: the first plane's, row's and column's residuals go
+//     to the previous bricks as they are formed;
+//   receive the next bricks' residuals; barrier.
+// Every word is written again only after the words it depends on came back, so
+// one slot per word suffices (the criterion's two sets alternate). Every wait
+// is bounded: after kWaitSpins loads without its word a work-group raises the abort
+// flag, every wait ends, and the host restores u and solves another way.
+//
+// The per-voxel arithmetic is cmf_voxel.h's, so the result equals the
+// per-iteration kernels' bit for bit; the criterion's sum is taken in another
+// order.
+#include <climits>
+#include <mutex>
+#include <vector>
+
+#include "cmf_onchip.h"
+#include "cmf_voxel.h"
+#include "mh_reduce.h"
+
+namespace {
+
+typedef unsigned long long Word;
+
+constexpr int kMaxThreads = 1024;
+constexpr int kMaxDevices = 64;
+constexpr int kWaitSpins = 1 << 16;  // loads of a word that does not come: about 50 ms
+constexpr int kCells = 1536;          // LDS cells of a tile and its faces
+constexpr int kRedFloats = 64;  // reduction scratch and the failure flag
+
+struct SumOp {
+    __device__ static float identity() { return 0.f; }
+    __device__ static float combine(float a, float b) { return a + b; }
+};
+
+// modes of the p-step
+constexpr int kAxial = 0;      // constant eigenvalues (l0, l1, l1)
+constexpr int kConst = 1;      // other constant eigenvalues
+constexpr int kPointwise = 2;  // eigenvalues of their own at every voxel
+
+struct Args {
+    const mh::OnchipSolve *solves;
+    int nsolves, nslots;
+    mh::OnchipFields F;
+    int d0, d1, d2;
+    int b1, b2, nt1, nt2, nz;
+    int num_iter, update;
+    float rcc, inv_rcc, rs0, rs1, rs2, ss0, ss1, ss2, error_bound, inv_n_rcc;
+    float sq0, sq1, sq2, rq0, rq1, rq2;
+    mh::AxiParams A;
+    Word *inbox;      // per brick: [z residuals | z h0 | in-plane residuals | in-plane h1, h2]
+    Word *parts;      // criterion partials, two sets per slot
+    int *abort;
+};
+
+template <int G>
+struct alignas(4 * G) Vec {
+    float v[G];
+};
+
+// Words are addressed by 32-bit byte offsets from the inbox (a few megabytes).
+__device__ __forceinline__ Word *word_at(Word *base, unsigned byte)
+{
+    return reinterpret_cast<Word *>(reinterpret_cast<char *>(base) + size_t(byte));
+}
+__device__ __forceinline__ Word ld_word(const Word *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_word(Word *p, unsigned tag, float v)
+{
+    __hip_atomic_store(p, (Word(tag) << 32) | __builtin_bit_cast(unsigned, v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Orders LDS accesses of the work-group around the barrier; global stores (the
+// words under way to other bricks) are not waited for.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The value of a word once its tag is `tag`; v is a first load of it. Gives up
+// when another work-group did or after kWaitSpins loads, raising both flags.
+__device__ __forceinline__ float wait_word(Word v, const Word *p, unsigned tag, int *abort, int *fail)
+{
+    for (int spin = 0; unsigned(v >> 32) != tag; ++spin) {
+        v = ld_word(p);
+        if ((spin & 15) == 15 && unsigned(v >> 32) != tag) {
+            if (spin > kWaitSpins ||
+                __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                *fail = 1;
+                break;
+            }
+        }
+    }
+    return __builtin_bit_cast(float, unsigned(v));
+}
+
+// A value the compiler cannot move computations on out of the loop (address
+// arithmetic hoisted out of it would hold a register per address).
+__device__ __forceinline__ unsigned here(unsigned v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+__device__ __forceinline__ int here_s(int v)  // the same for a uniform value
+{
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+template <int V, int MODE, bool SUP>
+__global__ void __launch_bounds__(kMaxThreads)
+cmf_onchip_kernel(const Args A)
+{
+    constexpr int G = V < 4 ? V : 4, NG = V / G;
+    constexpr int NF = MODE == kAxial ? 3 : MODE == kConst ? 4 : 7;
+    using VecG = Vec<G>;
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int t = int(threadIdx.x), NT = int(blockDim.x);
+    const int b1 = A.b1, b2 = A.b2, nc = b1 * b2;
+    // kCells cells each of the residual tile (own, the row after it, the column
+    // after it), of h1 (the row before it, own, a zero) and of h2 (own, the
+    // column before it, a zero); a cell holds G planes, NG tiles each
+    VecG *sT = reinterpret_cast<VecG *>(lds);
+    VecG *sH1 = sT + NG * kCells;
+    VecG *sH2 = sH1 + NG * kCells;
+    float *red = reinterpret_cast<float *>(sH2 + NG * kCells);
+    int *fail = reinterpret_cast<int *>(red + kRedFloats - 1);
+
+    const int per = A.nt1 * A.nt2 * A.nz;
+    const unsigned b = mh::xcd_block(blockIdx.x, gridDim.x);
+    const int slot = int(b) / per, lb = int(b) - slot * per;
+    const int bx = lb % A.nt2, by = (lb / A.nt2) % A.nt1, bz = lb / (A.nt1 * A.nt2);
+    const bool live = t < nc;
+    const int y = live ? t / b2 : 0, x = live ? t - y * b2 : 0, cell = live ? t : 0;
+    const int gy = by * b1 + y, gx = bx * b2 + x, z0 = bz * V;
+    const bool inv = live && gy < A.d1 && gx < A.d2;
+    const int nz = min(V, A.d0 - z0);
+    const int last0 = A.d0 - 1 - z0;  // the volume's last plane, counted from z0
+    const bool e1 = gy < A.d1 - 1, e2 = gx < A.d2 - 1;
+    const bool zp = z0 + V < A.d0, zm = bz > 0, yp = by + 1 < A.nt1, ym = by > 0,
+               xp = bx + 1 < A.nt2, xm = bx > 0;
+    const VecG *const tO = sT + cell;                                  // residual, own
+    const VecG *const t2 = sT + (x < b2 - 1 ? cell + 1 : nc + b2 + y);  // at +axis 2
+    const VecG *const m1p = sH1 + (inv ? cell : kCells - 1);            // h1 at -axis 1
+    const VecG *const m2p = sH2 + (inv ? (x > 0 ? cell - 1 : nc + y) : kCells - 1);
+
+    // words between bricks: byte offsets of this brick's inbox and of the parts
+    const int Wy = A.nt1 > 1 ? V * b2 : 0, Wx = A.nt2 > 1 ? V * b1 : 0, W = Wy + Wx;
+    const unsigned IB = 16u * unsigned(nc + W), box = b * IB, nc8 = 8u * unsigned(nc);
+    const unsigned boxT = box + 2u * nc8, boxH = boxT + 8u * unsigned(W);
+    const unsigned dz = unsigned(A.nt1 * A.nt2) * IB, dy = unsigned(A.nt2) * IB;
+    const unsigned x8 = 8u * unsigned(x), y8 = 8u * unsigned(y), t8 = 8u * unsigned(t);
+    const unsigned NT8 = 8u * unsigned(NT);
+    // in-plane faces this thread sends: residuals of the first row and column,
+    // h1 of the last row, h2 of the last column
+    const bool oTy = inv && y == 0 && ym, oTx = inv && x == 0 && xm;
+    const bool oHy = inv && y == b1 - 1 && yp, oHx = inv && x == b2 - 1 && xp;
+    // in-plane words this thread receives (words t and t + NT of the brick's)
+    // and the LDS floats they go to (-1: none)
+    int dT[2], dH[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int w = t + r * NT;
+        dT[r] = dH[r] = -1;
+        if (w < Wy) {
+            const int k = w / b2, xx = w - k * b2;
+            if (z0 + k < A.d0 && bx * b2 + xx < A.d2) {
+                if (yp) dT[r] = ((k / G) * kCells + nc + xx) * G + k % G;
+                if (ym) dH[r] = ((k / G) * kCells + xx) * G + k % G;
+            }
+        } else if (w < W) {
+            const int k = (w - Wy) / b1, yy = w - Wy - k * b1;
+            if (z0 + k < A.d0 && by * b1 + yy < A.d1) {
+                if (xp) dT[r] = ((k / G) * kCells + nc + b2 + yy) * G + k % G;
+                if (xm) dH[r] = (NG * kCells + (k / G) * kCells + nc + yy) * G + k % G;
+            }
+        }
+    }
+    float *fT = reinterpret_cast<float *>(sT), *fH = reinterpret_cast<float *>(sH1);
+
+    // the faces that have no neighbour, and the zero cells, stay zero
+    for (int i = t; i < 3 * NG * kCells * G + kRedFloats; i += NT) fT[i] = 0.f;
+    lds_barrier();
+
+    const unsigned st0 = unsigned(A.d1) * unsigned(A.d2);
+    const unsigned i0 = inv ? unsigned(z0) * st0 + unsigned(gy) * unsigned(A.d2) + unsigned(gx) : 0u;
+    unsigned tag = 1;
+    int nparts = 0;
+    for (int q = slot; q < A.nsolves; q += A.nslots) {
+        const mh::OnchipSolve S = A.solves[q];
+        float h0[V], h1[V], h2[V], pt[V], u[V], al[V], cs[V], ct[V], fr[V][NF];
+        unsigned lab = 0;
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            h0[k] = h1[k] = h2[k] = 0.f;
+            pt[k] = u[k] = al[k] = cs[k] = ct[k] = 0.f;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) fr[k][f] = 0.f;
+            if (MODE == kPointwise) fr[k][4] = fr[k][5] = fr[k][6] = 1.f;
+            if (inv && k < nz) {
+                const unsigned i = here(i0) + unsigned(k) * st0;
+                u[k] = S.u[i];
+                cs[k] = A.F.cs[i];
+                ct[k] = A.F.ct[i];
+                al[k] = S.alpha ? S.alpha[i] : S.w * expf(-S.gms[i] * S.k);
+                const float *e = A.F.eigs + (MODE == kPointwise ? 6u * i + 3u : 3u * i);
+                const mh::Quat qq = mh::expand_squeezed(e[0], e[1], e[2]);
+                if constexpr (MODE == kAxial) {
+                    mh::frame_axis(make_float4(qq.w, qq.x, qq.y, qq.z), fr[k][0], fr[k][1], fr[k][2]);
+                } else {
+                    fr[k][0] = qq.w;
+                    fr[k][1] = qq.x;
+                    fr[k][2] = qq.y;
+                    fr[k][3] = qq.z;
+                }
+                if constexpr (MODE == kPointwise) {
+                    fr[k][4] = e[-3];
+                    fr[k][5] = e[-2];
+                    fr[k][6] = e[-1];
+                }
+                if (SUP) lab |= unsigned(A.F.labels[i] & 3) << (2 * k);
+                pt[k] = fminf(cs[k], ct[k]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // the residuals the next bricks' p-steps take from this one: sent as
+        // plane k's are formed
+        auto send_T = [&](int k, float v) {
+            if (k == 0 && zm && inv) st_word(word_at(A.inbox, here(t8) + (box - dz)), tag, v);
+            if (k < here_s(nz)) {
+                if (oTy)
+                    st_word(word_at(A.inbox, here(x8) + (boxT - dy + unsigned(here_s(8 * b2) * k))), tag, v);
+                if (oTx)
+                    st_word(word_at(A.inbox,
+                                    here(y8) + (boxT - IB + 8u * unsigned(Wy) + unsigned(here_s(8 * b1) * k))),
+                            tag, v);
+            }
+        };
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            VecG T;
+#pragma unroll
+            for (int j = 0; j < G; ++j) {
+                const int k = g * G + j;
+                T.v[j] = inv && k < nz ? -(u[k] * A.rcc) : 0.f;
+                send_T(k, T.v[j]);
+            }
+            if (live) const_cast<VecG *>(tO)[g * kCells] = T;
+        }
+
+        int stop = 0, ncrit = 0;
+        for (int it = 0; it < A.num_iter; ++it) {
+            float zin = 0.f;
+            {
+                const bool rz = zp && inv;
+                const unsigned o = here(t8);
+                const Word *pz = word_at(A.inbox, o + box), *p0 = word_at(A.inbox, o + boxT),
+                           *p1 = word_at(A.inbox, o + (boxT + NT8));
+                Word vz = 0, v0 = 0, v1 = 0;
+                if (rz) vz = ld_word(pz);
+                if (dT[0] >= 0) v0 = ld_word(p0);
+                if (dT[1] >= 0) v1 = ld_word(p1);
+                if (dT[0] >= 0) fT[dT[0]] = wait_word(v0, p0, tag, A.abort, fail);
+                if (dT[1] >= 0) fT[dT[1]] = wait_word(v1, p1, tag, A.abort, fail);
+                if (rz) zin = wait_word(vz, pz, tag, A.abort, fail);
+            }
+            lds_barrier();
+            // p-step
+#pragma unroll
+            for (int g = NG - 1; g >= 0; --g) {
+                const VecG To = tO[g * kCells], T1 = tO[g * kCells + b2], T2 = t2[g * kCells];
+#pragma unroll
+                for (int j = G - 1; j >= 0; --j) {
+                    const int k = g * G + j;
+                    const float tn = j < G - 1 ? To.v[j < G - 1 ? j + 1 : j] : zin;
+                    const float g0 = k < here_s(last0) ? (tn - To.v[j]) * A.ss0 : 0.f;
+                    const float g1 = e1 ? (T1.v[j] - To.v[j]) * A.ss1 : 0.f;
+                    const float g2 = e2 ? (T2.v[j] - To.v[j]) * A.ss2 : 0.f;
+                    if constexpr (MODE == kAxial) {
+                        mh::cmf_p_voxel_axi(h0[k], h1[k], h2[k], g0, g1, g2, fr[k][0], fr[k][1],
+                                            fr[k][2], A.A, al[k]);
+                    } else {
+                        const mh::Mat3 R =
+                            mh::quat_to_mat(mh::Quat{fr[k][0], fr[k][1], fr[k][2], fr[k][3]});
+                        if constexpr (MODE == kConst)
+                            mh::cmf_p_voxel_m(h0[k], h1[k], h2[k], g0, g1, g2, R, A.sq0, A.sq1, A.sq2,
+                                              A.rq0, A.rq1, A.rq2, al[k]);
+                        else
+                            mh::cmf_p_voxel_m(h0[k], h1[k], h2[k], g0, g1, g2, R, fr[k][4], fr[k][5],
+                                              fr[k][6], 1.f / fr[k][4], 1.f / fr[k][5],
+                                              1.f / fr[k][6], al[k]);
+                    }
+                    if (k == V - 1 && zp && inv)
+                        st_word(word_at(A.inbox, here(t8) + (box + dz + nc8)), tag, h0[k]);
+                    if (k < here_s(nz)) {
+                        if (oHy)
+                            st_word(word_at(A.inbox, here(x8) + (boxH + dy + unsigned(here_s(8 * b2) * k))),
+                                    tag, h1[k]);
+                        if (oHx)
+                            st_word(word_at(A.inbox, here(y8) + (boxH + IB + 8u * unsigned(Wy) +
+                                                                 unsigned(here_s(8 * b1) * k))),
+                                    tag, h2[k]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                zin = To.v[0];
+                VecG w1, w2;
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    w1.v[j] = h1[g * G + j];
+                    w2.v[j] = h2[g * G + j];
+                }
+                if (live) {
+                    sH1[g * kCells + cell + b2] = w1;
+                    sH2[g * kCells + cell] = w2;
+                }
+            }
+            float below = 0.f;
+            {
+                const bool rz = zm && inv;
+                const unsigned o = here(t8);
+                const Word *pz = word_at(A.inbox, o + (box + nc8)), *p0 = word_at(A.inbox, o + boxH),
+                           *p1 = word_at(A.inbox, o + (boxH + NT8));
+                Word vz = 0, v0 = 0, v1 = 0;
+                if (rz) vz = ld_word(pz);
+                if (dH[0] >= 0) v0 = ld_word(p0);
+                if (dH[1] >= 0) v1 = ld_word(p1);
+                if (dH[0] >= 0) fH[dH[0]] = wait_word(v0, p0, tag, A.abort, fail);
+                if (dH[1] >= 0) fH[dH[1]] = wait_word(v1, p1, tag, A.abort, fail);
+                if (rz) below = wait_word(vz, pz, tag, A.abort, fail);
+            }
+            lds_barrier();
+            // u-step
+            ++tag;
+            const bool more = it + 1 < A.num_iter;
+            float aerr = 0.f;
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                const VecG m1 = m1p[g * kCells], m2 = m2p[g * kCells];
+                VecG T;
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    const int k = g * G + j;
+                    const float own0 = k < here_s(last0) ? h0[k] : 0.f;
+                    const float x0 = own0 - below;
+                    const float x1 = (e1 ? h1[k] : 0.f) - m1.v[j];
+                    const float x2 = (e2 ? h2[k] : 0.f) - m2.v[j];
+                    below = own0;
+                    const float div = mh::cmf_div(x0, x1, x2, A.rs0, A.rs1, A.rs2);
+                    float ub = 1.f, uf = 0.f;
+                    if (SUP) {
+                        uf = float((lab >> (2 * k)) & 1u);
+                        ub = ((lab >> (2 * k)) & 2u) ? 0.f : 1.f;
+                    }
+                    const float err = mh::cmf_u_voxel(div, pt[k], u[k], T.v[j], cs[k], ct[k], A.rcc,
+                                                      A.inv_rcc, ub, uf);
+                    aerr += fabsf(err);
+                    if (more) send_T(k, T.v[j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (live) const_cast<VecG *>(tO)[g * kCells] = T;
+            }
+            // the criterion: every work-group adds every brick's sum in the
+            // same order, so all of them take the same decision
+            if (it % A.update == 0) {
+                const int wv = t >> 6, nw = NT >> 6;
+                aerr = mh::wave_reduce<SumOp>(aerr);
+                if ((t & 63) == 0) red[wv] = aerr;
+                lds_barrier();
+                float s = 0.f;
+                for (int w = 0; w < nw; ++w) s += red[w];
+                if (per > 1) {
+                    Word *set = A.parts + (int64_t(slot) * 2 + (nparts & 1)) * per;
+                    ++nparts;
+                    if (t == 0) st_word(set + lb, tag, s);
+                    s = 0.f;
+                    for (int w = t; w < per; w += NT)
+                        s += wait_word(ld_word(set + w), set + w, tag, A.abort, fail);
+                    s = mh::wave_reduce<SumOp>(s);
+                    if ((t & 63) == 0) red[16 + wv] = s;
+                    lds_barrier();
+                    s = 0.f;
+                    for (int w = 0; w < nw; ++w) s += red[16 + w];
+                }
+                const float crit = s * A.inv_n_rcc;
+                if (lb == 0 && t == 0 && ncrit < S.crit_max) S.crit_log[ncrit] = crit;
+                ++ncrit;
+                if (crit != crit) stop = 1;
+                else if (crit < A.error_bound) stop = 2;
+                if (stop) break;
+            }
+        }
+        ++tag;
+        lds_barrier();
+        if (*fail) return;
+        if (inv) {
+#pragma unroll
+            for (int k = 0; k < V; ++k)
+                if (k < nz) S.u[i0 + unsigned(k) * st0] = u[k];
+        }
+        if (t == 0) {
+            if (lb == 0) {
+                *S.stop = stop;
+                *S.ncrit = ncrit;
+            }
+            atomicAdd(S.done, 1);
+        }
+    }
+}
+
+// The inbox and criterion words, the abort and done words to zero; u of every
+// solve kept in `keep`.
+__global__ void __launch_bounds__(mh::kBlock)
+onchip_prepare_kernel(Word *words, int64_t nwords, const mh::OnchipSolve *solves, int nsolves,
+                      int64_t n, float *keep, int *abort)
+{
+    const int64_t step = int64_t(gridDim.x) * blockDim.x;
+    const int64_t i0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    for (int64_t i = i0; i < nwords; i += step) words[i] = 0;
+    for (int q = 0; q < nsolves; ++q) {
+        const float *u = solves[q].u;
+        for (int64_t i = i0; i < n; i += step) keep[q * n + i] = u[i];
+    }
+    if (i0 < nsolves) *solves[i0].done = 0;
+    if (i0 == 0) *abort = 0;
+}
+
+__global__ void __launch_bounds__(mh::kBlock)
+onchip_restore_kernel(float *__restrict__ u, const float *__restrict__ keep, int64_t n)
+{
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n) u[i] = keep[i];
+}
+
+int64_t align256(int64_t b) { return (b + 255) & ~int64_t(255); }
+
+int mode_of(const mh_cmf_params *p)
+{
+    return !p->const_evals ? kPointwise : mh::axi_params(p).on ? kAxial : kConst;
+}
+
+int words_of(const mh::OnchipPlan &P)  // in-plane face words of a brick
+{
+    return (P.nt1 > 1 ? P.v * P.b2 : 0) + (P.nt2 > 1 ? P.v * P.b1 : 0);
+}
+
+int lds_of(const mh::OnchipPlan &P) { return 4 * (3 * P.v * kCells + kRedFloats); }
+
+int threads_of(const mh::OnchipPlan &P) { return (P.b1 * P.b2 + 63) / 64 * 64; }
+
+int compute_units(mh_ctx *ctx)
+{
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) {
+        (void)hipGetLastError();
+        cus = 0;
+    }
+    return cus;
+}
+
+template <int V, int MODE>
+const void *kernel_sup(bool sup)
+{
+    return sup ? reinterpret_cast<const void *>(&cmf_onchip_kernel<V, MODE, true>)
+               : reinterpret_cast<const void *>(&cmf_onchip_kernel<V, MODE, false>);
+}
+
+const void *kernel_of(int v, int mode, bool sup)
+{
+    switch (mode * 16 + v) {
+    case kAxial * 16 + 1: return kernel_sup<1, kAxial>(sup);
+    case kAxial * 16 + 2: return kernel_sup<2, kAxial>(sup);
+    case kAxial * 16 + 4: return kernel_sup<4, kAxial>(sup);
+    case kAxial * 16 + 8: return kernel_sup<8, kAxial>(sup);
+    case kConst * 16 + 1: return kernel_sup<1, kConst>(sup);
+    case kConst * 16 + 2: return kernel_sup<2, kConst>(sup);
+    case kConst * 16 + 4: return kernel_sup<4, kConst>(sup);
+    case kPointwise * 16 + 1: return kernel_sup<1, kPointwise>(sup);
+    case kPointwise * 16 + 2: return kernel_sup<2, kPointwise>(sup);
+    case kPointwise * 16 + 4: return kernel_sup<4, kPointwise>(sup);
+    default: return nullptr;
+    }
+}
+
+std::mutex g_device_mu[kMaxDevices];  // one on-chip launch per device at a time
+
+}  // namespace
+
+namespace mh {
+
+OnchipPlan onchip_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, int solves)
+{
+    OnchipPlan best;
+    const std::array<int, 5> key{dims[0], dims[1], dims[2], mode_of(prm), solves};
+    const auto f = ctx->onchip_plans.find(key);
+    if (f != ctx->onchip_plans.end()) {
+        const auto &c = f->second;
+        best.v = c[0], best.b1 = c[1], best.b2 = c[2], best.nt1 = c[3], best.nt2 = c[4], best.nz = c[5];
+        return best;
+    }
+    const int cus = ctx->device < kMaxDevices ? compute_units(ctx) : 0;
+    if (cus <= 0) return best;
+    const int vmax = mode_of(prm) == kAxial ? 8 : 4;
+    double best_cost = 0;
+    for (int v = 1; v <= vmax; v *= 2) {
+        const int nz = (dims[0] + v - 1) / v;
+        if (nz > cus) continue;
+        for (int n2 = 1; n2 <= std::min(dims[2], 16); ++n2) {
+            const int b2 = (dims[2] + n2 - 1) / n2;
+            if (b2 > kMaxThreads) continue;
+            const int least = (dims[1] + kMaxThreads / b2 - 1) / (kMaxThreads / b2);
+            for (int n1 = least; n1 <= std::min(dims[1], least + 16); ++n1) {
+                OnchipPlan P;
+                P.v = v;
+                P.b1 = (dims[1] + n1 - 1) / n1;
+                P.b2 = b2;
+                P.nt1 = (dims[1] + P.b1 - 1) / P.b1;
+                P.nt2 = (dims[2] + b2 - 1) / b2;
+                P.nz = nz;
+                if (P.blocks() > cus || words_of(P) > 2 * threads_of(P) ||
+                    P.b1 * P.b2 + P.b1 + P.b2 + 1 > kCells)
+                    continue;
+                // an iteration: the exchange, then issue of the waves of the
+                // busiest SIMD plane by plane
+                const int waves = (threads_of(P) / 64 + 3) / 4;
+                const double it = (P.blocks() > 1 ? 2.4 : 0.6) + 0.125 * v * waves +
+                                  0.3 * words_of(P) / 1024.0;
+                const int rounds = (solves + cus / P.blocks() - 1) / (cus / P.blocks());
+                if (best.v == 0 || it * rounds < best_cost) {
+                    best = P;
+                    best_cost = it * rounds;
+                }
+            }
+        }
+    }
+    ctx->onchip_plans[key] = {best.v, best.b1, best.b2, best.nt1, best.nt2, best.nz};
+    return best;
+}
+
+namespace {
+int slots_of(const OnchipPlan &P, int solves, int cus) { return std::min(solves, cus / P.blocks()); }
+int64_t nwords_of(const OnchipPlan &P, int slots)
+{
+    return int64_t(slots) * P.blocks() * (2 * (P.b1 * P.b2 + words_of(P)) + 2);
+}
+}  // namespace
+
+int64_t onchip_work_bytes(const OnchipPlan &P, int solves, int cus)
+{
+    if (P.v == 0) return 0;
+    return align256(sizeof(Word) * nwords_of(P, slots_of(P, solves, cus))) +
+           align256(sizeof(OnchipSolve) * int64_t(solves)) + 256;
+}
+
+int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int nsolves,
+               const OnchipFields &F, const int dims[3], const mh_cmf_params *prm, void *work,
+               int64_t work_bytes, hipStream_t s, bool *ran, std::vector<int> *finished)
+{
+    *ran = false;
+    if (finished) finished->clear();
+    const int64_t n = int64_t(dims[0]) * dims[1] * dims[2];
+    const int cus = compute_units(ctx), mode = mode_of(prm);
+    if (P.v == 0 || cus <= 0 || prm->num_iter < 1) return MH_OK;
+    if (int64_t(nsolves) * (int64_t(prm->num_iter) + 1) > INT_MAX / 2) return MH_OK;  // tags
+    const int64_t fixed = onchip_work_bytes(P, nsolves, cus);
+    if (work_bytes < fixed + int64_t(sizeof(float)) * n * nsolves) return MH_OK;
+    const void *kernel = kernel_of(P.v, mode, F.labels != nullptr);
+    if (!kernel) return MH_OK;
+    std::unique_lock<std::mutex> lock(g_device_mu[ctx->device], std::try_to_lock);
+    if (!lock.owns_lock()) return MH_OK;
+
+    const int slots = slots_of(P, nsolves, cus), lds = lds_of(P);
+    const int64_t nwords = nwords_of(P, slots);
+    char *base = static_cast<char *>(work);
+    Args A{};
+    A.inbox = reinterpret_cast<Word *>(base);
+    A.parts = A.inbox + nwords - int64_t(slots) * P.blocks() * 2;
+    base += align256(sizeof(Word) * nwords);
+    OnchipSolve *table = reinterpret_cast<OnchipSolve *>(base);
+    base += align256(sizeof(OnchipSolve) * int64_t(nsolves));
+    A.abort = reinterpret_cast<int *>(base);
+    float *keep = reinterpret_cast<float *>(base + 256);
+    A.solves = table;
+    A.nsolves = nsolves;
+    A.nslots = slots;
+    A.F = F;
+    A.d0 = dims[0];
+    A.d1 = dims[1];
+    A.d2 = dims[2];
+    A.b1 = P.b1;
+    A.b2 = P.b2;
+    A.nt1 = P.nt1;
+    A.nt2 = P.nt2;
+    A.nz = P.nz;
+    A.num_iter = prm->num_iter;
+    A.update = prm->update;
+    A.rcc = prm->rcc;
+    A.inv_rcc = float(1.0 / double(prm->rcc));
+    A.rs0 = prm->rs[0];
+    A.rs1 = prm->rs[1];
+    A.rs2 = prm->rs[2];
+    A.ss0 = prm->ss[0];
+    A.ss1 = prm->ss[1];
+    A.ss2 = prm->ss[2];
+    A.error_bound = prm->error_bound;
+    A.inv_n_rcc = float(1.0 / (double(n) * double(prm->rcc)));
+    A.sq0 = prm->sqev[0];
+    A.sq1 = prm->sqev[1];
+    A.sq2 = prm->sqev[2];
+    A.rq0 = float(1.0 / double(prm->sqev[0]));
+    A.rq1 = float(1.0 / double(prm->sqev[1]));
+    A.rq2 = float(1.0 / double(prm->sqev[2]));
+    A.A = axi_params(prm);
+    MH_CHECK(ctx, hipMemcpyAsync(table, solves, sizeof(OnchipSolve) * size_t(nsolves),
+                                 hipMemcpyHostToDevice, s));
+    const unsigned pb = unsigned(std::min<int64_t>(1024, blocks_for(std::max(n, nwords))));
+    hipLaunchKernelGGL(onchip_prepare_kernel, dim3(std::max(pb, blocks_for(nsolves))), dim3(kBlock), 0,
+                       s, A.inbox, nwords, table, nsolves, n, keep, A.abort);
+    MH_CHECK_LAUNCH(ctx, "onchip prepare");
+    void *args[] = {&A};
+    MH_CHECK(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(unsigned(slots * P.blocks())),
+                                                    dim3(unsigned(threads_of(P))), args,
+                                                    unsigned(lds), s);
+    if (e != hipSuccess) {  // the device does not hold every work-group: nothing ran
+        (void)hipGetLastError();
+        return MH_OK;
+    }
+    // every solve's done word counts the bricks that stored u
+    std::vector<int> done(static_cast<size_t>(nsolves), 0);
+    for (int q = 0; q < nsolves; ++q)
+        MH_CHECK(ctx, hipMemcpyAsync(&done[size_t(q)], solves[q].done, sizeof(int),
+                                     hipMemcpyDeviceToHost, s));
+    MH_CHECK(ctx, hipStreamSynchronize(s));
+    *ran = true;
+    for (int q = 0; q < nsolves; ++q) {
+        done[size_t(q)] = done[size_t(q)] == P.blocks();
+        if (done[size_t(q)]) continue;
+        *ran = false;
+        hipLaunchKernelGGL(onchip_restore_kernel, dim3(blocks_for(n)), dim3(kBlock), 0, s, solves[q].u,
+                           keep + q * n, n);
+        MH_CHECK_LAUNCH(ctx, "onchip restore");
+    }
+    if (finished) finished->swap(done);
+    return MH_OK;
+}
+
+}  // namespace mh

@@ -13,6 +13,7 @@
 #include <mutex>
 #include <vector>
 
+#include "cmf_onchip.h"
 #include "cmf_voxel.h"
 #include "mh_common.h"
 #include "mh_reduce.h"
@@ -20,7 +21,7 @@
 namespace {
 
 // control block (int32 words) at the head of the solver workspace
-enum : int { kStop = 0, kNcrit = 1, kCounter = 2, kParity = 3, kCtrlWords = 64 };
+enum : int { kStop = 0, kNcrit = 1, kCounter = 2, kParity = 3, kDone = 4, kCtrlWords = 64 };
 constexpr int kCritLogMax = 1 << 16;
 
 struct SumOp {
@@ -1596,6 +1597,27 @@ int solve_core(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, con
     return R.finish();
 }
 
+// The solve with its whole state on the chip, where the context's settings
+// leave the method open and the volume fits (the 128^3 cell: 2.7 times the
+// tuned sweep; the smallest volumes: twice the per-iteration kernels). Waits
+// for it; `ran` false: u is unchanged and nothing was done.
+int solve_onchip(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, const float *cs,
+                 const float *ct, const uint8_t *labels, const Dims D, int64_t n,
+                 const mh_cmf_params *prm, const Workspace &W, hipStream_t s, bool *ran)
+{
+    *ran = false;
+    if (ctx->sweep_mode != 0) return MH_OK;
+    const int dims[3] = {D.d0, D.d1, D.d2};
+    const mh::OnchipPlan P = mh::onchip_plan(ctx, dims, prm, 1);
+    if (P.v == 0) return MH_OK;
+    const mh::OnchipSolve S{u, alpha, nullptr, 0.f, 0.f, W.ctrl + kStop, W.ctrl + kNcrit, W.ctrl + kDone,
+                            W.crit_log, kCritLogMax};
+    char *room = reinterpret_cast<char *>(W.hp);  // the state arrays' room
+    const int64_t bytes = layout(n, nullptr, nullptr) - (room - reinterpret_cast<char *>(W.ctrl));
+    return mh::onchip_run(ctx, P, &S, 1, mh::OnchipFields{eigs, cs, ct, labels}, dims, prm, room, bytes,
+                          s, ran);
+}
+
 }  // namespace
 
 namespace {
@@ -1626,8 +1648,10 @@ MH_EXPORT int mh_cmf_solve(mh_ctx *ctx, float *u, const float *eigs, const float
     hipStream_t s = (hipStream_t)stream;
     const Dims D{int(dims[0]), int(dims[1]), int(dims[2])};
 
-    const int rc_core = solve_core(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, 1);
-    if (rc_core) return rc_core;
+    bool ran = false;
+    int rc = solve_onchip(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, &ran);
+    if (!rc && !ran) rc = solve_core(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, 1);
+    if (rc) return rc;
     return read_result(ctx, W, prm, res, crit_host, s);
 }
 
@@ -1813,12 +1837,16 @@ MH_EXPORT int mh_cmf_solve_noalloc(mh_ctx *ctx, float *u, const float *eigs, con
     layout(n, static_cast<char *>(ctx->noalloc_scratch), &W);
     hipStream_t s = (hipStream_t)stream;
     const Dims D{int(dims[0]), int(dims[1]), int(dims[2])};
+    bool ran = false;
+    int rc = solve_onchip(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, &ran);
+    if (rc) return rc;
+    if (ran) return read_result(ctx, W, prm, res, crit_host, s);
     // the method mh_cmf_solve tuned for these dims on this context, else the
     // untuned default; never tuned here (tuning creates events) and never
     // captured as a graph
     Runner R(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s);
     R.graphs_allowed = false;
-    int rc = R.init();
+    rc = R.init();
     if (rc) return rc;
     SweepMethod use;
     rc = R.choose(0, use);
@@ -2130,22 +2158,17 @@ MH_EXPORT int64_t mh_cmf_batched_workspace_bytes(int64_t n, int nsolves)
     return batch_layout(n, nsolves, kCritLogMax / 16, nullptr, nullptr);
 }
 
-MH_EXPORT int mh_cmf_solve_batched(mh_ctx *ctx, float *u, int S, const float *w_host,
-                                   const float *decay_host, const float *eigs, const float *gms,
-                                   const float *cs, const float *ct, const int64_t dims[3],
-                                   const mh_cmf_params *prm, void *work, int64_t work_bytes,
-                                   mh_cmf_result *res, void *stream)
+namespace {
+
+// The solves through the sweeps or the group kernels (mh_cmf_solve_batched's
+// arguments, checked there).
+int batched_swept(mh_ctx *ctx, float *u, int S, const float *w_host, const float *decay_host,
+                  const float *eigs, const float *gms, const float *cs, const float *ct,
+                  const int64_t dims[3], const mh_cmf_params *prm, void *work, mh_cmf_result *res,
+                  void *stream)
 {
-    MH_REQUIRE(ctx, mh::dims_ok(dims), "bad dims");
-    MH_REQUIRE(ctx, u && w_host && decay_host && eigs && gms && cs && ct && prm && work, "null pointer");
-    MH_REQUIRE(ctx, S >= 1, "nsolves must be >= 1");
-    MH_REQUIRE(ctx, prm->const_evals, "batched solves use constant eigenvalues");
-    MH_REQUIRE(ctx, prm->num_iter >= 0 && prm->update >= 1 && prm->rcc > 0.f, "bad params");
     const int maxcheck = maxcheck_for(prm);
-    MH_REQUIRE(ctx, maxcheck <= kCritLogMax / 16, "too many criterion checks (num_iter / update)");
     const int64_t n = dims[0] * dims[1] * dims[2];
-    MH_REQUIRE(ctx, work_bytes >= batch_layout(n, S, kCritLogMax / 16, nullptr, nullptr), "workspace too small");
-    MH_REQUIRE(ctx, (reinterpret_cast<uintptr_t>(work) & 255) == 0, "workspace must be 256-byte aligned");
     BatchWorkspace W;
     batch_layout(n, S, maxcheck, static_cast<char *>(work), &W);
     hipStream_t s = (hipStream_t)stream;
@@ -2397,6 +2420,103 @@ MH_EXPORT int mh_cmf_solve_batched(mh_ctx *ctx, float *u, int S, const float *w_
             res[j].iterations = st ? (stop[S + j] - 1) * prm->update + 1 : prm->num_iter;
             res[j].last_crit = nc > 0 ? log[int64_t(j) * maxcheck + nc - 1] : 0.f;
         }
+    }
+    return any_nan ? MH_STOPPED_NAN : MH_OK;
+}
+
+// Fills res[j] (may be null) from a solve's stop reason, number of criteria
+// and last criterion.
+void batched_result(mh_cmf_result *res, int stopped, int ncrit, float last, int maxcheck,
+                    const mh_cmf_params *prm)
+{
+    if (!res) return;
+    res->stopped = stopped;
+    res->ncrit = std::min(ncrit, maxcheck);
+    res->iterations = stopped ? (ncrit - 1) * prm->update + 1 : prm->num_iter;
+    res->last_crit = res->ncrit > 0 ? last : 0.f;
+}
+
+}  // namespace
+
+MH_EXPORT int mh_cmf_solve_batched(mh_ctx *ctx, float *u, int S, const float *w_host,
+                                   const float *decay_host, const float *eigs, const float *gms,
+                                   const float *cs, const float *ct, const int64_t dims[3],
+                                   const mh_cmf_params *prm, void *work, int64_t work_bytes,
+                                   mh_cmf_result *res, void *stream)
+{
+    MH_REQUIRE(ctx, mh::dims_ok(dims), "bad dims");
+    MH_REQUIRE(ctx, u && w_host && decay_host && eigs && gms && cs && ct && prm && work, "null pointer");
+    MH_REQUIRE(ctx, S >= 1, "nsolves must be >= 1");
+    MH_REQUIRE(ctx, prm->const_evals, "batched solves use constant eigenvalues");
+    MH_REQUIRE(ctx, prm->num_iter >= 0 && prm->update >= 1 && prm->rcc > 0.f, "bad params");
+    const int maxcheck = maxcheck_for(prm);
+    MH_REQUIRE(ctx, maxcheck <= kCritLogMax / 16, "too many criterion checks (num_iter / update)");
+    const int64_t n = dims[0] * dims[1] * dims[2];
+    MH_REQUIRE(ctx, work_bytes >= batch_layout(n, S, kCritLogMax / 16, nullptr, nullptr), "workspace too small");
+    MH_REQUIRE(ctx, (reinterpret_cast<uintptr_t>(work) & 255) == 0, "workspace must be 256-byte aligned");
+    hipStream_t s = (hipStream_t)stream;
+    auto swept = [&](int j, int count) {
+        return batched_swept(ctx, u + n * j, count, w_host + j, decay_host + j, eigs, gms, cs, ct, dims,
+                             prm, work, res ? res + j : nullptr, stream);
+    };
+    // with every setting automatic the solves stay on the chip where the
+    // volume fits, one after another or side by side
+    const bool automatic = ctx->sweep_mode == 0 && ctx->batch_sweep == 0 && ctx->batch_group == 0 &&
+                           ctx->batch_visit == 0;
+    const int idims[3] = {int(dims[0]), int(dims[1]), int(dims[2])};
+    mh::OnchipPlan P;
+    if (automatic) P = mh::onchip_plan(ctx, idims, prm, S);
+    if (P.v == 0) return swept(0, S);
+    int first = 0, any_nan = 0;
+    // volumes of the sweeps' range: the first pair tunes them for these dims
+    // (they run the solves when the device is shared with another on-chip
+    // solve), once per context
+    if (S > 2 && n >= 800000 && prm->num_iter >= 96 &&
+        ctx->sweep_tuned.find({idims[0], idims[1], idims[2]}) == ctx->sweep_tuned.end()) {
+        const int rc = swept(0, 2);
+        if (rc < 0) return rc;
+        any_nan |= rc == MH_STOPPED_NAN;
+        first = 2;
+    }
+    const int S1 = S - first;
+    BatchWorkspace W;
+    batch_layout(n, S, maxcheck, static_cast<char *>(work), &W);
+    std::vector<mh::OnchipSolve> solves(static_cast<size_t>(S1));
+    for (int j = 0; j < S1; ++j)
+        solves[size_t(j)] = mh::OnchipSolve{
+            u + n * (first + j), nullptr, gms, w_host[first + j],
+            float(1.0 / (double(decay_host[first + j]) * double(decay_host[first + j]))), W.stop + j,
+            W.ncrit + j, W.parity + j, W.crit_log + int64_t(j) * maxcheck, maxcheck};
+    char *room = reinterpret_cast<char *>(W.hp);
+    const int64_t bytes = work_bytes - (room - static_cast<char *>(work));
+    bool ran = false;
+    std::vector<int> done;
+    const int rc = mh::onchip_run(ctx, P, solves.data(), S1, mh::OnchipFields{eigs, cs, ct, nullptr}, idims,
+                                  prm, room, bytes, s, &ran, &done);
+    if (rc) return rc;
+    std::vector<int> ctrl(2 * size_t(S));
+    std::vector<float> log(size_t(S) * maxcheck);
+    if (std::any_of(done.begin(), done.end(), [](int d) { return d != 0; })) {
+        MH_CHECK(ctx, hipMemcpyAsync(ctrl.data(), W.stop, sizeof(int) * ctrl.size(), hipMemcpyDeviceToHost, s));
+        MH_CHECK(ctx, hipMemcpyAsync(log.data(), W.crit_log, sizeof(float) * log.size(),
+                                     hipMemcpyDeviceToHost, s));
+        MH_CHECK(ctx, hipStreamSynchronize(s));
+    }
+    for (int j = 0; j < S1; ++j) {
+        if (done.empty() || !done[size_t(j)]) {  // the rest of the solves one way or another
+            int count = 1;
+            while (j + count < S1 && (done.empty() || !done[size_t(j + count)])) ++count;
+            const int rcs = swept(first + j, count);
+            if (rcs < 0) return rcs;
+            any_nan |= rcs == MH_STOPPED_NAN;
+            j += count - 1;
+            continue;
+        }
+        const int st = ctrl[size_t(j)], nc = ctrl[size_t(S + j)];
+        any_nan |= st == 1;
+        batched_result(res ? res + first + j : nullptr, st, nc,
+                       nc > 0 ? log[size_t(j) * maxcheck + size_t(std::min(nc, maxcheck) - 1)] : 0.f,
+                       maxcheck, prm);
     }
     return any_nan ? MH_STOPPED_NAN : MH_OK;
 }

@@ -56,6 +56,8 @@ struct mh_ctx {
     // method the batched solver's tuner chose per volume dims (tile shape,
     // plane chunk), timed on pairs of solves
     std::map<std::array<int, 3>, std::pair<int, int>> batch_tuned;
+    // bricks of the on-chip solver per (dims, p-step form, solves)
+    std::map<std::array<int, 5>, std::array<int, 6>> onchip_plans;
     // resident work-groups of the sweep kernel on the device, per tile shape
     // (CU count x occupancy; 0 until queried)
     std::array<int, 16> sweep_slots{};
