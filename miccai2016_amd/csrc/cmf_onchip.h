@@ -10,9 +10,7 @@ namespace mh {
 // One solve of a set that shares dims, frames, capacities and parameters.
 struct OnchipSolve {
     float *u;            // u0 on entry, the labelling on exit
-    const float *alpha;  // or null: alpha = w exp(-gms k)
-    const float *gms;
-    float w, k;
+    const float *alpha;
     int *stop, *ncrit;   // device: stop reason and number of criteria
     int *done;           // device: set to 1 when u holds the result
     float *crit_log;     // device: crit_max values

@@ -40,11 +40,14 @@ namespace {
 
 typedef unsigned long long Word;
 
-constexpr int kMaxThreads = 1024;
 constexpr int kMaxDevices = 64;
-constexpr int kWaitSpins = 1 << 16;  // loads of a word that does not come: about 50 ms
-constexpr int kCells = 1536;          // LDS cells of a tile and its faces
-constexpr int kRedFloats = 64;  // reduction scratch and the failure flag
+constexpr int kWaitSpins = 1 << 16;  // loads of a word that does not come: tens of milliseconds
+constexpr int kRedFloats = 64;       // reduction scratch and the failure flag
+constexpr int kWords = 2;      // in-plane words a thread receives per phase
+
+constexpr int kMaxThreads = 1024;
+constexpr int kMaxPlanes = 8;  // per thread, constant eigenvalues (l0, l1, l1); else half
+constexpr int kCells = 1248;   // LDS cells of a tile and its faces
 
 struct SumOp {
     __device__ static float identity() { return 0.f; }
@@ -70,6 +73,13 @@ struct Args {
     Word *parts;      // criterion partials, two sets per slot
     int *abort;
 };
+
+// The sink of 8 planes is in LDS: 1024 threads have 128 registers each.
+constexpr bool sink_in_lds(int v) { return v == 8; }
+constexpr int lds_bytes(int v)
+{
+    return 4 * (3 * v * kCells + (sink_in_lds(v) ? v * kMaxThreads : 0) + kRedFloats);
+}
 
 template <int G>
 struct alignas(4 * G) Vec {
@@ -100,22 +110,16 @@ __device__ __forceinline__ void lds_barrier()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The value of a word once its tag is `tag`; v is a first load of it. Gives up
-// when another work-group did or after kWaitSpins loads, raising both flags.
-__device__ __forceinline__ float wait_word(Word v, const Word *p, unsigned tag, int *abort, int *fail)
+// Whether a wait ends without its word: every 16th load, when another
+// work-group gave up or after kWaitSpins loads. Raises both flags.
+__device__ __forceinline__ bool give_up(int spin, int *abort, int *fail)
 {
-    for (int spin = 0; unsigned(v >> 32) != tag; ++spin) {
-        v = ld_word(p);
-        if ((spin & 15) == 15 && unsigned(v >> 32) != tag) {
-            if (spin > kWaitSpins ||
-                __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-                __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                *fail = 1;
-                break;
-            }
-        }
-    }
-    return __builtin_bit_cast(float, unsigned(v));
+    if ((spin & 15) != 15) return false;
+    if (spin <= kWaitSpins && !__hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        return false;
+    __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *fail = 1;
+    return true;
 }
 
 // A value the compiler cannot move computations on out of the loop (address
@@ -138,17 +142,19 @@ cmf_onchip_kernel(const Args A)
 {
     constexpr int G = V < 4 ? V : 4, NG = V / G;
     constexpr int NF = MODE == kAxial ? 3 : MODE == kConst ? 4 : 7;
+    constexpr int kTile = NG * kCells;  // LDS vectors of one field
+    constexpr bool kCsLds = sink_in_lds(V);
     using VecG = Vec<G>;
     extern __shared__ __align__(16) unsigned char lds[];
     const int t = int(threadIdx.x), NT = int(blockDim.x);
     const int b1 = A.b1, b2 = A.b2, nc = b1 * b2;
-    // kCells cells each of the residual tile (own, the row after it, the column
-    // after it), of h1 (the row before it, own, a zero) and of h2 (own, the
-    // column before it, a zero); a cell holds G planes, NG tiles each
+    // LDS: the residual, h1 and h2 tiles, NG of kCells vectors of G planes
+    // each. Cells: the brick's own [0, nc), the row beyond it [nc, nc + b2)
+    // (after it for the residual, before it for h1), the column beyond it
+    // [nc + b2, nc + b2 + b1) (h2's lies in h1's tile), and a zero at the end.
     VecG *sT = reinterpret_cast<VecG *>(lds);
-    VecG *sH1 = sT + NG * kCells;
-    VecG *sH2 = sH1 + NG * kCells;
-    float *red = reinterpret_cast<float *>(sH2 + NG * kCells);
+    float *fT = reinterpret_cast<float *>(sT);
+    float *red = fT + (3 * kTile + (kCsLds ? NG * kMaxThreads : 0)) * G;
     int *fail = reinterpret_cast<int *>(red + kRedFloats - 1);
 
     const int per = A.nt1 * A.nt2 * A.nz;
@@ -164,136 +170,157 @@ cmf_onchip_kernel(const Args A)
     const bool e1 = gy < A.d1 - 1, e2 = gx < A.d2 - 1;
     const bool zp = z0 + V < A.d0, zm = bz > 0, yp = by + 1 < A.nt1, ym = by > 0,
                xp = bx + 1 < A.nt2, xm = bx > 0;
-    const VecG *const tO = sT + cell;                                  // residual, own
-    const VecG *const t2 = sT + (x < b2 - 1 ? cell + 1 : nc + b2 + y);  // at +axis 2
-    const VecG *const m1p = sH1 + (inv ? cell : kCells - 1);            // h1 at -axis 1
-    const VecG *const m2p = sH2 + (inv ? (x > 0 ? cell - 1 : nc + y) : kCells - 1);
+    VecG *const own = sT + cell;
+    const VecG *const t2 = sT + (x < b2 - 1 ? cell + 1 : nc + b2 + y);  // residual at +axis 2
+    const VecG *const m1p =                                             // h1 at -axis 1
+        sT + kTile + (!inv ? kCells - 1 : y > 0 ? cell - b2 : nc + x);
+    const VecG *const m2p =                                             // h2 at -axis 2
+        sT + (!inv ? kTile + kCells - 1 : x > 0 ? 2 * kTile + cell - 1 : kTile + nc + b2 + y);
 
-    // words between bricks: byte offsets of this brick's inbox and of the parts
+    // words between bricks: byte offsets of this brick's inbox and of its parts
     const int Wy = A.nt1 > 1 ? V * b2 : 0, Wx = A.nt2 > 1 ? V * b1 : 0, W = Wy + Wx;
     const unsigned IB = 16u * unsigned(nc + W), box = b * IB, nc8 = 8u * unsigned(nc);
     const unsigned boxT = box + 2u * nc8, boxH = boxT + 8u * unsigned(W);
     const unsigned dz = unsigned(A.nt1 * A.nt2) * IB, dy = unsigned(A.nt2) * IB;
     const unsigned x8 = 8u * unsigned(x), y8 = 8u * unsigned(y), t8 = 8u * unsigned(t);
     const unsigned NT8 = 8u * unsigned(NT);
-    // in-plane faces this thread sends: residuals of the first row and column,
-    // h1 of the last row, h2 of the last column
-    const bool oTy = inv && y == 0 && ym, oTx = inv && x == 0 && xm;
-    const bool oHy = inv && y == b1 - 1 && yp, oHx = inv && x == b2 - 1 && xp;
-    // in-plane words this thread receives (words t and t + NT of the brick's)
-    // and the LDS floats they go to (-1: none)
-    int dT[2], dH[2];
+    // faces this thread sends: residuals of the first plane, row and column,
+    // h0 of the last plane, h1 of the last row, h2 of the last column; the
+    // waves that send whole rows run first in their phase
+    const bool oTz = inv && zm, oTy = inv && y == 0 && ym, oTx = inv && x == 0 && xm;
+    const bool oHz = inv && zp, oHy = inv && y == b1 - 1 && yp, oHx = inv && x == b2 - 1 && xp;
+    const bool firstT = __any(oTy), firstH = __any(oHy);
+    // in-plane words this thread receives (words t, t + NT, .. of the brick's)
+    // and the LDS floats they go to, in the residual's tile or h1's
+    constexpr int R = kWords;
+    int d[R];
+    bool rT[R], rH[R];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
+    for (int r = 0; r < R; ++r) {
         const int w = t + r * NT;
-        dT[r] = dH[r] = -1;
-        if (w < Wy) {
-            const int k = w / b2, xx = w - k * b2;
-            if (z0 + k < A.d0 && bx * b2 + xx < A.d2) {
-                if (yp) dT[r] = ((k / G) * kCells + nc + xx) * G + k % G;
-                if (ym) dH[r] = ((k / G) * kCells + xx) * G + k % G;
-            }
-        } else if (w < W) {
-            const int k = (w - Wy) / b1, yy = w - Wy - k * b1;
-            if (z0 + k < A.d0 && by * b1 + yy < A.d1) {
-                if (xp) dT[r] = ((k / G) * kCells + nc + b2 + yy) * G + k % G;
-                if (xm) dH[r] = (NG * kCells + (k / G) * kCells + nc + yy) * G + k % G;
-            }
-        }
+        const bool isy = w < Wy;
+        const int div = isy ? b2 : b1, v = isy ? w : w - Wy, k = v / div, i = v - k * div;
+        const bool in = w < W && k < nz && (isy ? bx * b2 + i < A.d2 : by * b1 + i < A.d1);
+        d[r] = ((k / G) * kCells + nc + (isy ? 0 : b2) + i) * G + k % G;
+        rT[r] = in && (isy ? yp : xp);
+        rH[r] = in && (isy ? ym : xm);
     }
-    float *fT = reinterpret_cast<float *>(sT), *fH = reinterpret_cast<float *>(sH1);
 
     // the faces that have no neighbour, and the zero cells, stay zero
-    for (int i = t; i < 3 * NG * kCells * G + kRedFloats; i += NT) fT[i] = 0.f;
+    for (int i = t; i < lds_bytes(V) / 4; i += NT) fT[i] = 0.f;
     lds_barrier();
+
+    // Receives this thread's words: one load of each as its phase ends, then
+    // all of them again until none is missing. (The first load half a phase
+    // earlier mostly came too early: 5.6 against 4.9 us per iteration at
+    // 128^3.) The axis-0 neighbour's value is returned, the in-plane ones go to
+    // `tile`.
+    Word first[R + 1];
+    auto look = [&](unsigned zoff, bool rz, unsigned off, const bool (&rv)[R]) {
+        const unsigned o = here(t8);
+        first[R] = 0;
+        if (rz) first[R] = ld_word(word_at(A.inbox, o + zoff));
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            first[r] = 0;
+            if (rv[r]) first[r] = ld_word(word_at(A.inbox, o + (off + unsigned(r) * NT8)));
+        }
+    };
+    auto receive = [&](unsigned zoff, bool rz, unsigned off, const bool (&rv)[R], float *tile,
+                       unsigned tag) {
+        for (int spin = 0;; ++spin) {
+            bool missing = rz && unsigned(first[R] >> 32) != tag;
+#pragma unroll
+            for (int r = 0; r < R; ++r) missing |= rv[r] && unsigned(first[r] >> 32) != tag;
+            if (!missing || give_up(spin, A.abort, fail)) break;
+            look(zoff, rz, off, rv);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (rv[r]) tile[d[r]] = __builtin_bit_cast(float, unsigned(first[r]));
+        return rz ? __builtin_bit_cast(float, unsigned(first[R])) : 0.f;
+    };
+    // sends planes [g G, g G + G) of a row or a column
+    auto send_row = [&](bool mine, unsigned v8, unsigned off, int stride, int g, const float (&v)[G],
+                        unsigned tag) {
+        if (!mine) return;
+        const unsigned o = here(v8) + off;
+#pragma unroll
+        for (int j = 0; j < G; ++j)
+            if (g * G + j < here_s(nz))
+                st_word(word_at(A.inbox, o + unsigned(here_s(8 * stride) * (g * G + j))), tag, v[j]);
+    };
 
     const unsigned st0 = unsigned(A.d1) * unsigned(A.d2);
     const unsigned i0 = inv ? unsigned(z0) * st0 + unsigned(gy) * unsigned(A.d2) + unsigned(gx) : 0u;
     unsigned tag = 1;
     int nparts = 0;
     for (int q = slot; q < A.nsolves; q += A.nslots) {
-        const mh::OnchipSolve S = A.solves[q];
         float h0[V], h1[V], h2[V], pt[V], u[V], al[V], cs[V], ct[V], fr[V][NF];
         unsigned lab = 0;
+        {
+            const mh::OnchipSolve S = A.solves[q];
 #pragma unroll
-        for (int k = 0; k < V; ++k) {
-            h0[k] = h1[k] = h2[k] = 0.f;
-            pt[k] = u[k] = al[k] = cs[k] = ct[k] = 0.f;
+            for (int k = 0; k < V; ++k) {
+                h0[k] = h1[k] = h2[k] = 0.f;
+                pt[k] = u[k] = al[k] = cs[k] = ct[k] = 0.f;
 #pragma unroll
-            for (int f = 0; f < NF; ++f) fr[k][f] = 0.f;
-            if (MODE == kPointwise) fr[k][4] = fr[k][5] = fr[k][6] = 1.f;
-            if (inv && k < nz) {
-                const unsigned i = here(i0) + unsigned(k) * st0;
-                u[k] = S.u[i];
-                cs[k] = A.F.cs[i];
-                ct[k] = A.F.ct[i];
-                al[k] = S.alpha ? S.alpha[i] : S.w * expf(-S.gms[i] * S.k);
-                const float *e = A.F.eigs + (MODE == kPointwise ? 6u * i + 3u : 3u * i);
-                const mh::Quat qq = mh::expand_squeezed(e[0], e[1], e[2]);
-                if constexpr (MODE == kAxial) {
-                    mh::frame_axis(make_float4(qq.w, qq.x, qq.y, qq.z), fr[k][0], fr[k][1], fr[k][2]);
-                } else {
-                    fr[k][0] = qq.w;
-                    fr[k][1] = qq.x;
-                    fr[k][2] = qq.y;
-                    fr[k][3] = qq.z;
+                for (int f = 0; f < NF; ++f) fr[k][f] = 0.f;
+                if (MODE == kPointwise) fr[k][4] = fr[k][5] = fr[k][6] = 1.f;
+                if (inv && k < nz) {
+                    const unsigned i = here(i0) + unsigned(k) * st0;
+                    u[k] = S.u[i];
+                    cs[k] = A.F.cs[i];
+                    ct[k] = A.F.ct[i];
+                    al[k] = S.alpha[i];
+                    const float *e = A.F.eigs + (MODE == kPointwise ? 6u * i + 3u : 3u * i);
+                    const mh::Quat qq = mh::expand_squeezed(e[0], e[1], e[2]);
+                    if constexpr (MODE == kAxial) {
+                        mh::frame_axis(make_float4(qq.w, qq.x, qq.y, qq.z), fr[k][0], fr[k][1], fr[k][2]);
+                    } else {
+                        fr[k][0] = qq.w;
+                        fr[k][1] = qq.x;
+                        fr[k][2] = qq.y;
+                        fr[k][3] = qq.z;
+                    }
+                    if constexpr (MODE == kPointwise) {
+                        fr[k][4] = e[-3];
+                        fr[k][5] = e[-2];
+                        fr[k][6] = e[-1];
+                    }
+                    if (SUP) lab |= unsigned(A.F.labels[i] & 3) << (2 * k);
+                    pt[k] = fminf(cs[k], ct[k]);
                 }
-                if constexpr (MODE == kPointwise) {
-                    fr[k][4] = e[-3];
-                    fr[k][5] = e[-2];
-                    fr[k][6] = e[-1];
-                }
-                if (SUP) lab |= unsigned(A.F.labels[i] & 3) << (2 * k);
-                pt[k] = fminf(cs[k], ct[k]);
             }
-            __builtin_amdgcn_sched_barrier(0);
         }
-        // the residuals the next bricks' p-steps take from this one: sent as
-        // plane k's are formed
-        auto send_T = [&](int k, float v) {
-            if (k == 0 && zm && inv) st_word(word_at(A.inbox, here(t8) + (box - dz)), tag, v);
-            if (k < here_s(nz)) {
-                if (oTy)
-                    st_word(word_at(A.inbox, here(x8) + (boxT - dy + unsigned(here_s(8 * b2) * k))), tag, v);
-                if (oTx)
-                    st_word(word_at(A.inbox,
-                                    here(y8) + (boxT - IB + 8u * unsigned(Wy) + unsigned(here_s(8 * b1) * k))),
-                            tag, v);
-            }
-        };
+        // the first residuals
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
             VecG T;
 #pragma unroll
-            for (int j = 0; j < G; ++j) {
-                const int k = g * G + j;
-                T.v[j] = inv && k < nz ? -(u[k] * A.rcc) : 0.f;
-                send_T(k, T.v[j]);
+            for (int j = 0; j < G; ++j) T.v[j] = inv && g * G + j < nz ? -(u[g * G + j] * A.rcc) : 0.f;
+            if (g == 0 && oTz) st_word(word_at(A.inbox, here(t8) + (box - dz)), tag, T.v[0]);
+            send_row(oTy, x8, boxT - dy, b2, g, T.v, tag);
+            send_row(oTx, y8, boxT - IB + 8u * unsigned(Wy), b1, g, T.v, tag);
+            if (live) own[g * kCells] = T;
+            if (kCsLds && live) {
+#pragma unroll
+                for (int j = 0; j < G; ++j) T.v[j] = cs[g * G + j];
+                own[3 * kTile + g * kMaxThreads] = T;
             }
-            if (live) const_cast<VecG *>(tO)[g * kCells] = T;
         }
+        look(box, oHz, boxT, rT);
 
         int stop = 0, ncrit = 0;
         for (int it = 0; it < A.num_iter; ++it) {
-            float zin = 0.f;
-            {
-                const bool rz = zp && inv;
-                const unsigned o = here(t8);
-                const Word *pz = word_at(A.inbox, o + box), *p0 = word_at(A.inbox, o + boxT),
-                           *p1 = word_at(A.inbox, o + (boxT + NT8));
-                Word vz = 0, v0 = 0, v1 = 0;
-                if (rz) vz = ld_word(pz);
-                if (dT[0] >= 0) v0 = ld_word(p0);
-                if (dT[1] >= 0) v1 = ld_word(p1);
-                if (dT[0] >= 0) fT[dT[0]] = wait_word(v0, p0, tag, A.abort, fail);
-                if (dT[1] >= 0) fT[dT[1]] = wait_word(v1, p1, tag, A.abort, fail);
-                if (rz) zin = wait_word(vz, pz, tag, A.abort, fail);
-            }
+            float zin = receive(box, oHz, boxT, rT, fT, tag);
             lds_barrier();
             // p-step
+            if (firstH) __builtin_amdgcn_s_setprio(2);
 #pragma unroll
             for (int g = NG - 1; g >= 0; --g) {
-                const VecG To = tO[g * kCells], T1 = tO[g * kCells + b2], T2 = t2[g * kCells];
+                const VecG To = own[g * kCells], T1 = own[g * kCells + b2], T2 = t2[g * kCells];
+                VecG w1, w2;
 #pragma unroll
                 for (int j = G - 1; j >= 0; --j) {
                     const int k = g * G + j;
@@ -305,64 +332,43 @@ cmf_onchip_kernel(const Args A)
                         mh::cmf_p_voxel_axi(h0[k], h1[k], h2[k], g0, g1, g2, fr[k][0], fr[k][1],
                                             fr[k][2], A.A, al[k]);
                     } else {
-                        const mh::Mat3 R =
+                        const mh::Mat3 M =
                             mh::quat_to_mat(mh::Quat{fr[k][0], fr[k][1], fr[k][2], fr[k][3]});
                         if constexpr (MODE == kConst)
-                            mh::cmf_p_voxel_m(h0[k], h1[k], h2[k], g0, g1, g2, R, A.sq0, A.sq1, A.sq2,
+                            mh::cmf_p_voxel_m(h0[k], h1[k], h2[k], g0, g1, g2, M, A.sq0, A.sq1, A.sq2,
                                               A.rq0, A.rq1, A.rq2, al[k]);
                         else
-                            mh::cmf_p_voxel_m(h0[k], h1[k], h2[k], g0, g1, g2, R, fr[k][4], fr[k][5],
+                            mh::cmf_p_voxel_m(h0[k], h1[k], h2[k], g0, g1, g2, M, fr[k][4], fr[k][5],
                                               fr[k][6], 1.f / fr[k][4], 1.f / fr[k][5],
                                               1.f / fr[k][6], al[k]);
                     }
-                    if (k == V - 1 && zp && inv)
+                    w1.v[j] = h1[k];
+                    w2.v[j] = h2[k];
+                    if (k == V - 1 && oHz)
                         st_word(word_at(A.inbox, here(t8) + (box + dz + nc8)), tag, h0[k]);
-                    if (k < here_s(nz)) {
-                        if (oHy)
-                            st_word(word_at(A.inbox, here(x8) + (boxH + dy + unsigned(here_s(8 * b2) * k))),
-                                    tag, h1[k]);
-                        if (oHx)
-                            st_word(word_at(A.inbox, here(y8) + (boxH + IB + 8u * unsigned(Wy) +
-                                                                 unsigned(here_s(8 * b1) * k))),
-                                    tag, h2[k]);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
                 }
                 zin = To.v[0];
-                VecG w1, w2;
-#pragma unroll
-                for (int j = 0; j < G; ++j) {
-                    w1.v[j] = h1[g * G + j];
-                    w2.v[j] = h2[g * G + j];
-                }
+                send_row(oHy, x8, boxH + dy, b2, g, w1.v, tag);
+                send_row(oHx, y8, boxH + IB + 8u * unsigned(Wy), b1, g, w2.v, tag);
                 if (live) {
-                    sH1[g * kCells + cell + b2] = w1;
-                    sH2[g * kCells + cell] = w2;
+                    own[kTile + g * kCells] = w1;
+                    own[2 * kTile + g * kCells] = w2;
                 }
             }
-            float below = 0.f;
-            {
-                const bool rz = zm && inv;
-                const unsigned o = here(t8);
-                const Word *pz = word_at(A.inbox, o + (box + nc8)), *p0 = word_at(A.inbox, o + boxH),
-                           *p1 = word_at(A.inbox, o + (boxH + NT8));
-                Word vz = 0, v0 = 0, v1 = 0;
-                if (rz) vz = ld_word(pz);
-                if (dH[0] >= 0) v0 = ld_word(p0);
-                if (dH[1] >= 0) v1 = ld_word(p1);
-                if (dH[0] >= 0) fH[dH[0]] = wait_word(v0, p0, tag, A.abort, fail);
-                if (dH[1] >= 0) fH[dH[1]] = wait_word(v1, p1, tag, A.abort, fail);
-                if (rz) below = wait_word(vz, pz, tag, A.abort, fail);
-            }
+            look(box + nc8, oTz, boxH, rH);
+            if (firstH) __builtin_amdgcn_s_setprio(0);
+            float below = receive(box + nc8, oTz, boxH, rH, fT + kTile * G, tag);
             lds_barrier();
             // u-step
             ++tag;
+            if (firstT) __builtin_amdgcn_s_setprio(2);
             const bool more = it + 1 < A.num_iter;
             float aerr = 0.f;
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
                 const VecG m1 = m1p[g * kCells], m2 = m2p[g * kCells];
-                VecG T;
+                VecG T, C;
+                if (kCsLds) C = own[3 * kTile + g * kMaxThreads];
 #pragma unroll
                 for (int j = 0; j < G; ++j) {
                     const int k = g * G + j;
@@ -374,22 +380,27 @@ cmf_onchip_kernel(const Args A)
                     const float div = mh::cmf_div(x0, x1, x2, A.rs0, A.rs1, A.rs2);
                     float ub = 1.f, uf = 0.f;
                     if (SUP) {
-                        uf = float((lab >> (2 * k)) & 1u);
-                        ub = ((lab >> (2 * k)) & 2u) ? 0.f : 1.f;
+                        const unsigned l = here(lab) >> (2 * k);
+                        uf = float(l & 1u);
+                        ub = (l & 2u) ? 0.f : 1.f;
                     }
-                    const float err = mh::cmf_u_voxel(div, pt[k], u[k], T.v[j], cs[k], ct[k], A.rcc,
+                    const float err = mh::cmf_u_voxel(div, pt[k], u[k], T.v[j], kCsLds ? C.v[j] : cs[k], ct[k], A.rcc,
                                                       A.inv_rcc, ub, uf);
                     aerr += fabsf(err);
-                    if (more) send_T(k, T.v[j]);
-                    __builtin_amdgcn_sched_barrier(0);
+                    if (k == 0 && more && oTz)
+                        st_word(word_at(A.inbox, here(t8) + (box - dz)), tag, T.v[0]);
                 }
-                if (live) const_cast<VecG *>(tO)[g * kCells] = T;
+                send_row(oTy && more, x8, boxT - dy, b2, g, T.v, tag);
+                send_row(oTx && more, y8, boxT - IB + 8u * unsigned(Wy), b1, g, T.v, tag);
+                if (live) own[g * kCells] = T;
             }
+            if (more) look(box, oHz, boxT, rT);
+            if (firstT) __builtin_amdgcn_s_setprio(0);
             // the criterion: every work-group adds every brick's sum in the
             // same order, so all of them take the same decision
             if (it % A.update == 0) {
                 const int wv = t >> 6, nw = NT >> 6;
-                aerr = mh::wave_reduce<SumOp>(aerr);
+                aerr = mh::wave_reduce<SumOp>(inv ? aerr : 0.f);
                 if ((t & 63) == 0) red[wv] = aerr;
                 lds_barrier();
                 float s = 0.f;
@@ -399,8 +410,14 @@ cmf_onchip_kernel(const Args A)
                     ++nparts;
                     if (t == 0) st_word(set + lb, tag, s);
                     s = 0.f;
-                    for (int w = t; w < per; w += NT)
-                        s += wait_word(ld_word(set + w), set + w, tag, A.abort, fail);
+                    for (int w = t; w < per; w += NT) {
+                        Word v = ld_word(set + w);
+                        for (int spin = 0; unsigned(v >> 32) != tag; ++spin) {
+                            if (give_up(spin, A.abort, fail)) break;
+                            v = ld_word(set + w);
+                        }
+                        s += __builtin_bit_cast(float, unsigned(v));
+                    }
                     s = mh::wave_reduce<SumOp>(s);
                     if ((t & 63) == 0) red[16 + wv] = s;
                     lds_barrier();
@@ -408,7 +425,10 @@ cmf_onchip_kernel(const Args A)
                     for (int w = 0; w < nw; ++w) s += red[16 + w];
                 }
                 const float crit = s * A.inv_n_rcc;
-                if (lb == 0 && t == 0 && ncrit < S.crit_max) S.crit_log[ncrit] = crit;
+                if (lb == 0 && t == 0) {
+                    const mh::OnchipSolve &S = A.solves[here_s(q)];
+                    if (ncrit < S.crit_max) S.crit_log[ncrit] = crit;
+                }
                 ++ncrit;
                 if (crit != crit) stop = 1;
                 else if (crit < A.error_bound) stop = 2;
@@ -418,10 +438,12 @@ cmf_onchip_kernel(const Args A)
         ++tag;
         lds_barrier();
         if (*fail) return;
+        const mh::OnchipSolve &S = A.solves[here_s(q)];
         if (inv) {
+            float *out = S.u;
 #pragma unroll
             for (int k = 0; k < V; ++k)
-                if (k < nz) S.u[i0 + unsigned(k) * st0] = u[k];
+                if (k < nz) out[i0 + unsigned(k) * st0] = u[k];
         }
         if (t == 0) {
             if (lb == 0) {
@@ -469,8 +491,6 @@ int words_of(const mh::OnchipPlan &P)  // in-plane face words of a brick
     return (P.nt1 > 1 ? P.v * P.b2 : 0) + (P.nt2 > 1 ? P.v * P.b1 : 0);
 }
 
-int lds_of(const mh::OnchipPlan &P) { return 4 * (3 * P.v * kCells + kRedFloats); }
-
 int threads_of(const mh::OnchipPlan &P) { return (P.b1 * P.b2 + 63) / 64 * 64; }
 
 int compute_units(mh_ctx *ctx)
@@ -507,6 +527,27 @@ const void *kernel_of(int v, int mode, bool sup)
     }
 }
 
+bool plan_fits(const mh::OnchipPlan &P)
+{
+    const int nc = P.b1 * P.b2;
+    return nc <= kMaxThreads && words_of(P) <= kWords * threads_of(P) && nc + P.b1 + P.b2 + 1 <= kCells;
+}
+
+// Microseconds of an iteration, from measured plans (8 planes of 8 x 128
+// voxels per brick 4.9, of 8 x 64 3.4; 4 of 10 x 96 3.7, of 8 x 64 2.6; 2 of
+// 8 x 64 2.6; 1 of 10 x 37 2.3, of 16 x 64 3.4; bricks split along axis 2: 8 of
+// 16 x 64 6.3, 4 of 32 x 32 4.8): the two exchanges, the issue of a SIMD's waves
+// plane by plane (one wave alone does not hide its own latencies), the axis-0
+// words where little work covers them, and along a split axis 2 the words every
+// wave sends last.
+double iteration_us(const mh::OnchipPlan &P)
+{
+    if (P.blocks() == 1) return 0.8 + 0.1 * P.v * ((threads_of(P) + 255) / 256);
+    const int waves = (threads_of(P) + 255) / 256;
+    return 2.0 + 0.09 * P.v * (waves == 1 && P.v > 1 ? 3 : waves) +
+           (P.v < 4 ? 0.6 * P.b1 * P.b2 / 1024.0 : 0.0) + (P.nt2 > 1 ? 0.22 * P.v : 0.0);
+}
+
 std::mutex g_device_mu[kMaxDevices];  // one on-chip launch per device at a time
 
 }  // namespace
@@ -525,7 +566,7 @@ OnchipPlan onchip_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm,
     }
     const int cus = ctx->device < kMaxDevices ? compute_units(ctx) : 0;
     if (cus <= 0) return best;
-    const int vmax = mode_of(prm) == kAxial ? 8 : 4;
+    const int vmax = mode_of(prm) == kAxial ? kMaxPlanes : kMaxPlanes / 2;
     double best_cost = 0;
     for (int v = 1; v <= vmax; v *= 2) {
         const int nz = (dims[0] + v - 1) / v;
@@ -542,18 +583,12 @@ OnchipPlan onchip_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm,
                 P.nt1 = (dims[1] + P.b1 - 1) / P.b1;
                 P.nt2 = (dims[2] + b2 - 1) / b2;
                 P.nz = nz;
-                if (P.blocks() > cus || words_of(P) > 2 * threads_of(P) ||
-                    P.b1 * P.b2 + P.b1 + P.b2 + 1 > kCells)
-                    continue;
-                // an iteration: the exchange, then issue of the waves of the
-                // busiest SIMD plane by plane
-                const int waves = (threads_of(P) / 64 + 3) / 4;
-                const double it = (P.blocks() > 1 ? 2.4 : 0.6) + 0.125 * v * waves +
-                                  0.3 * words_of(P) / 1024.0;
+                if (P.blocks() > cus || !plan_fits(P)) continue;
                 const int rounds = (solves + cus / P.blocks() - 1) / (cus / P.blocks());
-                if (best.v == 0 || it * rounds < best_cost) {
+                const double cost = iteration_us(P) * rounds;
+                if (best.v == 0 || cost < best_cost) {
                     best = P;
-                    best_cost = it * rounds;
+                    best_cost = cost;
                 }
             }
         }
@@ -594,7 +629,7 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     std::unique_lock<std::mutex> lock(g_device_mu[ctx->device], std::try_to_lock);
     if (!lock.owns_lock()) return MH_OK;
 
-    const int slots = slots_of(P, nsolves, cus), lds = lds_of(P);
+    const int slots = slots_of(P, nsolves, cus), lds = lds_bytes(P.v);
     const int64_t nwords = nwords_of(P, slots);
     char *base = static_cast<char *>(work);
     Args A{};

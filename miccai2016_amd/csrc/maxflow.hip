@@ -1610,8 +1610,8 @@ int solve_onchip(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, c
     const int dims[3] = {D.d0, D.d1, D.d2};
     const mh::OnchipPlan P = mh::onchip_plan(ctx, dims, prm, 1);
     if (P.v == 0) return MH_OK;
-    const mh::OnchipSolve S{u, alpha, nullptr, 0.f, 0.f, W.ctrl + kStop, W.ctrl + kNcrit, W.ctrl + kDone,
-                            W.crit_log, kCritLogMax};
+    const mh::OnchipSolve S{u, alpha, W.ctrl + kStop, W.ctrl + kNcrit, W.ctrl + kDone, W.crit_log,
+                            kCritLogMax};
     char *room = reinterpret_cast<char *>(W.hp);  // the state arrays' room
     const int64_t bytes = layout(n, nullptr, nullptr) - (room - reinterpret_cast<char *>(W.ctrl));
     return mh::onchip_run(ctx, P, &S, 1, mh::OnchipFields{eigs, cs, ct, labels}, dims, prm, room, bytes,
@@ -2483,12 +2483,25 @@ MH_EXPORT int mh_cmf_solve_batched(mh_ctx *ctx, float *u, int S, const float *w_
     batch_layout(n, S, maxcheck, static_cast<char *>(work), &W);
     std::vector<mh::OnchipSolve> solves(static_cast<size_t>(S1));
     for (int j = 0; j < S1; ++j)
-        solves[size_t(j)] = mh::OnchipSolve{
-            u + n * (first + j), nullptr, gms, w_host[first + j],
-            float(1.0 / (double(decay_host[first + j]) * double(decay_host[first + j]))), W.stop + j,
-            W.ncrit + j, W.parity + j, W.crit_log + int64_t(j) * maxcheck, maxcheck};
-    char *room = reinterpret_cast<char *>(W.hp);
-    const int64_t bytes = work_bytes - (room - static_cast<char *>(work));
+        solves[size_t(j)] =
+            mh::OnchipSolve{u + n * (first + j), W.pt + n * j, W.stop + j, W.ncrit + j, W.parity + j,
+                            W.crit_log + int64_t(j) * maxcheck, maxcheck};
+    // every solve's alpha, where its pt would be, by the kernel that forms it
+    // for the sweeps (the exponential rounds as the compiler contracts it)
+    for (int j = 0; j < S1; j += kSI) {
+        SolveParams sp{};
+        const int count = std::min(kSI, S1 - j);
+        for (int k = 0; k < count; ++k) {
+            const double d = decay_host[first + j + k];
+            sp.w[k] = w_host[first + j + k];
+            sp.k[k] = float(1.0 / (d * d));
+        }
+        hipLaunchKernelGGL(cmf_group_alpha_kernel, dim3(mh::blocks_for(n), count), dim3(mh::kBlock), 0,
+                           s, gms, n, sp, W.pt + n * j);
+    }
+    MH_CHECK_LAUNCH(ctx, "batched alpha");
+    char *room = reinterpret_cast<char *>(W.hp);  // the room of hp
+    const int64_t bytes = reinterpret_cast<char *>(W.pt) - room;
     bool ran = false;
     std::vector<int> done;
     const int rc = mh::onchip_run(ctx, P, solves.data(), S1, mh::OnchipFields{eigs, cs, ct, nullptr}, idims,
