@@ -376,7 +376,10 @@ int mh_cmf_batched_set_sweep(mh_ctx *ctx, int mode);
  * reference). In mode 0 (default) a solve whose volume fits the device's
  * registers (about 2^21 voxels with constant eigenvalues (l0, l1, l1), half
  * of that otherwise) stays on the chip from its first iteration to its last,
- * unless another such solve is running on the device; what follows is for the
+ * unless another such solve is running on the device. On the same condition a
+ * larger one with eigenvalues (l0, l1, l1) goes through the volume with a
+ * sliding window of planes, up to 31 iterations a pass, where that is faster
+ * (measured: 256^3 1.8 times, with seeds 3.8 times). What follows is for the
  * others. Unsupervised constant-eigenvalue solves may advance two, three
  * or four iterations per pass over the state (temporal blocking along axis
  * 0; tile shapes 1-5 two levels, 6-7 three, 8-9 four). mode 0

@@ -34,14 +34,13 @@
 
 #include "cmf_onchip.h"
 #include "cmf_voxel.h"
+#include "cmf_words.h"
 #include "mh_reduce.h"
 
 namespace {
 
-typedef unsigned long long Word;
+using namespace mh;
 
-constexpr int kMaxDevices = 64;
-constexpr int kWaitSpins = 1 << 16;  // loads of a word that does not come: tens of milliseconds
 constexpr int kRedFloats = 64;       // three sets of the waves' sums, the failure flag last
 constexpr int kWords = 2;      // in-plane words a thread receives per phase
 
@@ -82,61 +81,6 @@ constexpr int lds_bytes(int v, int mode)
 {
     return 4 * (3 * v * kCells + kRedFloats +
                 (caps_in_lds(v, mode) ? (v + 4) * kMaxThreads : 0));
-}
-
-template <int G>
-struct alignas(4 * G) Vec {
-    float v[G];
-};
-
-// Words are addressed by 32-bit byte offsets from the inbox (a few megabytes).
-__device__ __forceinline__ Word *word_at(Word *base, unsigned byte)
-{
-    return reinterpret_cast<Word *>(reinterpret_cast<char *>(base) + size_t(byte));
-}
-__device__ __forceinline__ Word ld_word(const Word *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_word(Word *p, unsigned tag, float v)
-{
-    __hip_atomic_store(p, (Word(tag) << 32) | __builtin_bit_cast(unsigned, v), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Orders LDS accesses of the work-group around the barrier; global stores (the
-// words under way to other bricks) are not waited for.
-__device__ __forceinline__ void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// Whether a wait ends without its word: every 16th load, when another
-// work-group gave up or after kWaitSpins loads. Raises both flags.
-__device__ __forceinline__ bool give_up(int spin, int *abort, int *fail)
-{
-    if ((spin & 15) != 15) return false;
-    if (spin <= kWaitSpins && !__hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        return false;
-    __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *fail = 1;
-    return true;
-}
-
-// A value the compiler cannot move computations on out of the loop (address
-// arithmetic hoisted out of it would hold a register per address).
-__device__ __forceinline__ unsigned here(unsigned v)
-{
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
-__device__ __forceinline__ int here_s(int v)  // the same for a uniform value
-{
-    asm volatile("" : "+s"(v));
-    return v;
 }
 
 template <int V, int MODE, bool SUP, bool DEFER>
@@ -618,11 +562,13 @@ double iteration_us(const mh::OnchipPlan &P)
            (P.v < 4 ? 0.6 * P.b1 * P.b2 / 1024.0 : 0.0) + (P.nt2 > 1 ? 0.22 * P.v : 0.0);
 }
 
-std::mutex g_device_mu[kMaxDevices];  // one on-chip launch per device at a time
+std::mutex g_device_mu[kMaxDevices];
 
 }  // namespace
 
 namespace mh {
+
+std::mutex &device_lock(int device) { return g_device_mu[device]; }
 
 OnchipPlan onchip_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, int solves)
 {
@@ -696,7 +642,7 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     if (work_bytes < fixed + int64_t(sizeof(float)) * n * nsolves) return MH_OK;
     const void *kernel = kernel_of(P.v, mode, F.labels != nullptr, prm->update);
     if (!kernel) return MH_OK;
-    std::unique_lock<std::mutex> lock(g_device_mu[ctx->device], std::try_to_lock);
+    std::unique_lock<std::mutex> lock(device_lock(ctx->device), std::try_to_lock);
     if (!lock.owns_lock()) return MH_OK;
 
     const int slots = slots_of(P, nsolves, cus), lds = lds_bytes(P.v, mode);

@@ -14,14 +14,17 @@
 #include <vector>
 
 #include "cmf_onchip.h"
+#include "cmf_slide.h"
 #include "cmf_voxel.h"
+#include "cmf_words.h"
 #include "mh_common.h"
 #include "mh_reduce.h"
 
 namespace {
 
 // control block (int32 words) at the head of the solver workspace
-enum : int { kStop = 0, kNcrit = 1, kCounter = 2, kParity = 3, kDone = 4, kCtrlWords = 64 };
+enum : int { kStop = 0, kNcrit = 1, kCounter = 2, kParity = 3, kDone = 4, kAbort = 5, kAbortIt = 6,
+             kAbortCur = 7, kCtrlWords = 64 };
 constexpr int kCritLogMax = 1 << 16;
 
 struct SumOp {
@@ -235,6 +238,7 @@ constexpr SweepShape kSweepShapes[] = {{12, 64, 1024, 2}, {11, 32, 512, 2}, {4, 
                                        {27, 27, 1024, 3}, {9, 57, 1024, 4},  {25, 25, 1024, 4}};
 constexpr int kNumSweepShapes = 9;
 constexpr int kShape3 = 5;  // the three-level shape of a four-level method's three-level passes
+constexpr int kSlideShape = 100;  // not a tile shape: the sliding passes (cmf_slide.hip)
 constexpr int kDefaultShape = 6;  // untuned solves: the 27 x 27 three-level shape
 // iterations timed per candidate method (after a warm-up pass): shorter
 // windows let launch-to-launch noise of a few per cent pick a slower shape
@@ -1256,7 +1260,7 @@ __global__ void __launch_bounds__(mh::kBlock)
 cmf_sweep_final_kernel(float *__restrict__ u, const float *__restrict__ u2, int64_t n,
                        const int *__restrict__ ctrl)
 {
-    if (ctrl[kParity] != 1) return;
+    if (ctrl[kParity] != 1 || ctrl[kStop] == mh::kSlideAborted) return;
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) u[i] = u2[i];
 }
@@ -1299,6 +1303,15 @@ int64_t layout(int64_t n, char *base, Workspace *w)
     return off;
 }
 
+// Control words of a solve whose sliding pass could not be completed, as they
+// were before it.
+__global__ void slide_resume_kernel(int *ctrl, int cur)
+{
+    ctrl[kStop] = 0;
+    ctrl[kAbort] = 0;
+    ctrl[kParity] = cur;
+}
+
 __global__ void zero_ints(int *p, int n)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1331,7 +1344,18 @@ struct Runner {
     int cur = 0, it = 0, limit = 0;
     bool swept = false;
     bool graphs_allowed = true;  // false: never capture (no stream or graph is created)
+    // Sliding passes: allowed to a caller that waits for the solve with this
+    // Runner alive (it holds the device's lock until then), taken by choose.
+    bool may_slide = false;
+    mh::SlidePlan slide;
+    int slide_rc = 0;  // of the last sliding pass: after an error the solve goes on without
+    std::unique_lock<std::mutex> slide_lock;
 
+    Runner(Runner &&) = default;
+    ~Runner()  // also after an error the lock is held until the last pass is done
+    {
+        if (slide_lock.owns_lock()) (void)hipStreamSynchronize(s);
+    }
     Runner(mh_ctx *c, float *u_, const float *e, const float *a, const float *cs_, const float *ct_,
            const uint8_t *l, Dims d, int64_t n_, const mh_cmf_params *p, const Workspace &w,
            hipStream_t st)
@@ -1354,6 +1378,51 @@ struct Runner {
                            W.hp, W.pt, W.tmp, u, cs, ct, n, prm->rcc);
         MH_CHECK_LAUNCH(ctx, "cmf init");
         return MH_OK;
+    }
+
+    // Takes the sliding passes for this solve if they pay, the device is free
+    // of other launches whose work-groups wait for one another and there is
+    // room for their words.
+    int try_slide(bool *taken)
+    {
+        *taken = false;
+        const int dims[3] = {D.d0, D.d1, D.d2};
+        slide = mh::slide_plan(ctx, dims, prm, sup);
+        if (slide.levels == 0) return MH_OK;
+        slide_lock = std::unique_lock<std::mutex>(mh::device_lock(ctx->device), std::try_to_lock);
+        if (!slide_lock.owns_lock()) return MH_OK;
+        const size_t bytes = size_t(mh::slide_inbox_bytes(slide));
+        if (ctx->slide_bytes < bytes) {
+            if (ctx->slide_inbox) (void)hipFree(ctx->slide_inbox);
+            ctx->slide_inbox = nullptr;
+            ctx->slide_bytes = 0;
+            ctx->slide_tags = 0;
+            if (hipMalloc(&ctx->slide_inbox, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                ctx->slide_inbox = nullptr;
+                slide_lock.unlock();
+                return MH_OK;
+            }
+            ctx->slide_bytes = bytes;
+        }
+        *taken = true;
+        return MH_OK;
+    }
+
+    int slide_step(int lv, bool chk)
+    {
+        const int dims[3] = {D.d0, D.d1, D.d2};
+        mh::SlideFields F{W.hp, W.tmp, W.pt, u, W.hp2, W.tmp2, W.pt2, W.u2, W.q4, alpha, cs, ct, labels};
+        if (cur) {
+            std::swap(const_cast<float *&>(F.hp), F.hpo);
+            std::swap(const_cast<float *&>(F.tmp), F.tmpo);
+            std::swap(const_cast<float *&>(F.pt), F.pto);
+            std::swap(const_cast<float *&>(F.u), F.uo);
+        }
+        const mh::SlideControl C{W.ctrl + kStop, W.ctrl + kParity, W.ctrl + kAbort, W.ctrl + kAbortIt,
+                                 W.ctrl + kAbortCur};
+        return mh::slide_pass(ctx, slide, F, dims, prm, lv, it, chk, cur, C, W.partials,
+                              ctx->slide_inbox, &ctx->slide_tags, s);
     }
 
     int64_t sweep_grid_of(const SweepMethod &m) const
@@ -1381,6 +1450,24 @@ struct Runner {
     // does not go past `limit`; returns the iterations advanced
     int step(const SweepMethod &m)
     {
+        if (m.shape == kSlideShape) {
+            const int lv = sweep_levels(slide.levels, it, std::min(prm->num_iter, limit), prm->update);
+            // passes of one or two levels: a sweep, with seeds an iteration
+            if (lv < 3 || slide_rc) {
+                const SweepMethod sweep{0, model_zchunk(0)};
+                return step(!sup && usable(sweep) ? sweep : SweepMethod{-1, 0});
+            }
+            const bool chk = ((it + lv - 1) % prm->update) == 0;
+            slide_rc = slide_step(lv, chk);
+            if (slide_rc) return 0;  // nothing was launched
+            if (chk)
+                hipLaunchKernelGGL(cmf_crit_kernel, dim3(1), dim3(1024), 0, s, W.partials, slide.blocks(),
+                                   UP.inv_n_rcc, UP.error_bound, W.ctrl, W.crit_log);
+            cur ^= 1;
+            swept = true;
+            it += lv;
+            return lv;
+        }
         if (m.shape < 0) {
             float *hp = cur ? W.hp2 : W.hp, *tmp = cur ? W.tmp2 : W.tmp;
             float *pt = cur ? W.pt2 : W.pt, *uu = cur ? W.u2 : u;
@@ -1442,6 +1529,15 @@ struct Runner {
     {
         use = SweepMethod{-1, 0};
         const std::array<int, 3> key{D.d0, D.d1, D.d2};
+        if (may_slide && ctx->sweep_mode == 0) {
+            bool taken = false;
+            const int rc = try_slide(&taken);
+            if (rc) return rc;
+            if (taken) {
+                use = SweepMethod{kSlideShape, 0};
+                return MH_OK;
+            }
+        }
         if (ctx->sweep_mode == 1 || !sweep_elig) return MH_OK;
         if (ctx->sweep_mode == 2) {
             const int k = ctx->sweep_shape > 0 ? std::min(ctx->sweep_shape, kNumSweepShapes) - 1 : 0;
@@ -1621,6 +1717,7 @@ int solve_onchip(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, c
 }  // namespace
 
 namespace {
+constexpr int kResumeSolve = 1 << 20;  // read_result: a sliding pass was not completed
 int read_result(mh_ctx *ctx, const Workspace &W, const mh_cmf_params *prm, mh_cmf_result *res,
                 float *crit_host, hipStream_t s);
 }  // namespace
@@ -1650,9 +1747,30 @@ MH_EXPORT int mh_cmf_solve(mh_ctx *ctx, float *u, const float *eigs, const float
 
     bool ran = false;
     int rc = solve_onchip(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, &ran);
-    if (!rc && !ran) rc = solve_core(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, 1);
     if (rc) return rc;
-    return read_result(ctx, W, prm, res, crit_host, s);
+    if (ran) return read_result(ctx, W, prm, res, crit_host, s);
+    Runner R(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s);
+    R.may_slide = true;
+    rc = R.init();
+    for (;;) {
+        SweepMethod use;
+        if (!rc) rc = R.choose(1, use);
+        if (!rc) rc = R.run_until(use, prm->num_iter);
+        if (!rc) rc = R.finish();
+        if (!rc) rc = read_result(ctx, W, prm, res, crit_host, s);
+        if (rc != kResumeSolve) return rc;
+        // a sliding pass gave up waiting for a part of the device: from its
+        // input on, which is as it was, the solve takes the other methods
+        int at[2];
+        MH_CHECK(ctx, hipMemcpy(at, W.ctrl + kAbortIt, sizeof(at), hipMemcpyDeviceToHost));
+        R.may_slide = false;
+        R.slide_lock.unlock();
+        R.it = at[0];
+        R.cur = at[1];
+        hipLaunchKernelGGL(slide_resume_kernel, dim3(1), dim3(1), 0, s, W.ctrl, R.cur);
+        MH_CHECK_LAUNCH(ctx, "cmf resume");
+        rc = MH_OK;
+    }
 }
 
 namespace {
@@ -1664,6 +1782,7 @@ int read_result(mh_ctx *ctx, const Workspace &W, const mh_cmf_params *prm, mh_cm
     int ctrl[kCtrlWords];
     MH_CHECK(ctx, hipMemcpyAsync(ctrl, W.ctrl, sizeof(ctrl), hipMemcpyDeviceToHost, s));
     MH_CHECK(ctx, hipStreamSynchronize(s));
+    if (ctrl[kStop] == mh::kSlideAborted) return kResumeSolve;
     const int ncrit = std::min(ctrl[kNcrit], kCritLogMax);
     float last = 0.f;
     if (ncrit > 0)

@@ -58,6 +58,11 @@ struct mh_ctx {
     std::map<std::array<int, 3>, std::pair<int, int>> batch_tuned;
     // bricks of the on-chip solver per (dims, p-step form, solves)
     std::map<std::array<int, 5>, std::array<int, 6>> onchip_plans;
+    // words the work-groups of the sliding passes exchange (grown on demand),
+    // and the last tag used in them
+    void *slide_inbox = nullptr;
+    size_t slide_bytes = 0;
+    unsigned slide_tags = 0;
     // resident work-groups of the sweep kernel on the device, per tile shape
     // (CU count x occupancy; 0 until queried)
     std::array<int, 16> sweep_slots{};
