@@ -40,10 +40,12 @@ int64_t onchip_work_bytes(const OnchipPlan &plan, int solves, int max_blocks);
 // Enqueue the solves on `s` and wait for them. `ran`: every solve has its
 // result. Otherwise (the device runs another on-chip solve, or could not hold
 // every work-group at once) `finished`, empty or one flag per solve, says
-// which have; u of the others is as it was.
+// which have; u of the others is as it was. One solve may ask for `head`:
+// head_bytes from its stop word on, its done word among them, come with the
+// same transfer.
 int onchip_run(mh_ctx *ctx, const OnchipPlan &plan, const OnchipSolve *solves, int nsolves,
                const OnchipFields &F, const int dims[3], const mh_cmf_params *prm, void *work,
                int64_t work_bytes, hipStream_t s, bool *ran,
-               std::vector<int> *finished = nullptr);
+               std::vector<int> *finished = nullptr, void *head = nullptr, size_t head_bytes = 0);
 
 }  // namespace mh

@@ -28,6 +28,7 @@
 // The per-voxel arithmetic is cmf_voxel.h's, so the result equals the
 // per-iteration kernels' bit for bit; the criterion's sum is taken in another
 // order.
+#include <algorithm>
 #include <climits>
 #include <mutex>
 #include <vector>
@@ -462,12 +463,20 @@ cmf_onchip_kernel(const Args A)
     }
 }
 
+// A few solves reach the device as an argument: a transfer of their table costs
+// the host 10 us.
+constexpr int kFew = 16;
+struct Few {
+    mh::OnchipSolve s[kFew];
+};
+
 // The inbox and criterion words, the abort and done words to zero; u of every
-// solve kept in `keep`.
+// solve kept in `keep`; the table of a few solves.
 __global__ void __launch_bounds__(mh::kBlock)
-onchip_prepare_kernel(Word *words, int64_t nwords, const mh::OnchipSolve *solves, int nsolves,
+onchip_prepare_kernel(Word *words, int64_t nwords, mh::OnchipSolve *table, const Few few, int nsolves,
                       int64_t n, float *keep, int *abort)
 {
+    const mh::OnchipSolve *solves = nsolves <= kFew ? few.s : table;
     const int64_t step = int64_t(gridDim.x) * blockDim.x;
     const int64_t i0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     for (int64_t i = i0; i < nwords; i += step) words[i] = 0;
@@ -475,7 +484,10 @@ onchip_prepare_kernel(Word *words, int64_t nwords, const mh::OnchipSolve *solves
         const float *u = solves[q].u;
         for (int64_t i = i0; i < n; i += step) keep[q * n + i] = u[i];
     }
-    if (i0 < nsolves) *solves[i0].done = 0;
+    if (i0 < nsolves) {
+        *solves[i0].done = 0;
+        if (nsolves <= kFew) table[i0] = solves[i0];
+    }
     if (i0 == 0) *abort = 0;
 }
 
@@ -630,7 +642,8 @@ int64_t onchip_work_bytes(const OnchipPlan &P, int solves, int cus)
 
 int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int nsolves,
                const OnchipFields &F, const int dims[3], const mh_cmf_params *prm, void *work,
-               int64_t work_bytes, hipStream_t s, bool *ran, std::vector<int> *finished)
+               int64_t work_bytes, hipStream_t s, bool *ran, std::vector<int> *finished, void *head,
+               size_t head_bytes)
 {
     *ran = false;
     if (finished) finished->clear();
@@ -687,11 +700,15 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     A.rq1 = float(1.0 / double(prm->sqev[1]));
     A.rq2 = float(1.0 / double(prm->sqev[2]));
     A.A = axi_params(prm);
-    MH_CHECK(ctx, hipMemcpyAsync(table, solves, sizeof(OnchipSolve) * size_t(nsolves),
-                                 hipMemcpyHostToDevice, s));
+    Few few{};
+    if (nsolves <= kFew)
+        std::copy(solves, solves + nsolves, few.s);
+    else
+        MH_CHECK(ctx, hipMemcpyAsync(table, solves, sizeof(OnchipSolve) * size_t(nsolves),
+                                     hipMemcpyHostToDevice, s));
     const unsigned pb = unsigned(std::min<int64_t>(1024, blocks_for(std::max(n, nwords))));
     hipLaunchKernelGGL(onchip_prepare_kernel, dim3(std::max(pb, blocks_for(nsolves))), dim3(kBlock), 0,
-                       s, A.inbox, nwords, table, nsolves, n, keep, A.abort);
+                       s, A.inbox, nwords, table, few, nsolves, n, keep, A.abort);
     MH_CHECK_LAUNCH(ctx, "onchip prepare");
     void *args[] = {&A};
     MH_CHECK(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
@@ -704,10 +721,14 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     }
     // every solve's done word counts the bricks that stored u
     std::vector<int> done(static_cast<size_t>(nsolves), 0);
-    for (int q = 0; q < nsolves; ++q)
-        MH_CHECK(ctx, hipMemcpyAsync(&done[size_t(q)], solves[q].done, sizeof(int),
-                                     hipMemcpyDeviceToHost, s));
+    if (head)
+        MH_CHECK(ctx, hipMemcpyAsync(head, solves[0].stop, head_bytes, hipMemcpyDeviceToHost, s));
+    else
+        for (int q = 0; q < nsolves; ++q)
+            MH_CHECK(ctx, hipMemcpyAsync(&done[size_t(q)], solves[q].done, sizeof(int),
+                                         hipMemcpyDeviceToHost, s));
     MH_CHECK(ctx, hipStreamSynchronize(s));
+    if (head) done[0] = static_cast<const int *>(head)[solves[0].done - solves[0].stop];
     *ran = true;
     for (int q = 0; q < nsolves; ++q) {
         done[size_t(q)] = done[size_t(q)] == P.blocks();

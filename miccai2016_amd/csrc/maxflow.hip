@@ -1277,6 +1277,21 @@ struct Workspace {
     float *hp2, *pt2, *tmp2, *u2;
 };
 
+// The host's copy of a solve's control words and first criteria, which lie side
+// by side at the head of the workspace: one transfer brings both (a transfer
+// of a few bytes costs the host 10 to 15 us).
+constexpr int kHostCrit = 960;
+struct HostResult {
+    int ctrl[kCtrlWords];
+    float crit[kHostCrit];
+    static size_t bytes(const mh_cmf_params *prm)
+    {
+        const int64_t crits = (int64_t(prm->num_iter) + prm->update - 1) / prm->update;
+        return sizeof(int) * kCtrlWords + sizeof(float) * size_t(std::min<int64_t>(crits, kHostCrit));
+    }
+};
+static_assert(sizeof(int) * kCtrlWords == 256, "criteria follow the control words");
+
 int64_t align256(int64_t b) { return (b + 255) & ~int64_t(255); }
 
 int64_t layout(int64_t n, char *base, Workspace *w)
@@ -1699,7 +1714,7 @@ int solve_core(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, con
 // for it; `ran` false: u is unchanged and nothing was done.
 int solve_onchip(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, const float *cs,
                  const float *ct, const uint8_t *labels, const Dims D, int64_t n,
-                 const mh_cmf_params *prm, const Workspace &W, hipStream_t s, bool *ran)
+                 const mh_cmf_params *prm, const Workspace &W, hipStream_t s, HostResult *got, bool *ran)
 {
     *ran = false;
     if (ctx->sweep_mode != 0) return MH_OK;
@@ -1711,7 +1726,7 @@ int solve_onchip(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, c
     char *room = reinterpret_cast<char *>(W.hp);  // the state arrays' room
     const int64_t bytes = layout(n, nullptr, nullptr) - (room - reinterpret_cast<char *>(W.ctrl));
     return mh::onchip_run(ctx, P, &S, 1, mh::OnchipFields{eigs, cs, ct, labels}, dims, prm, room, bytes,
-                          s, ran);
+                          s, ran, nullptr, got, got->bytes(prm));
 }
 
 }  // namespace
@@ -1719,7 +1734,7 @@ int solve_onchip(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, c
 namespace {
 constexpr int kResumeSolve = 1 << 20;  // read_result: a sliding pass was not completed
 int read_result(mh_ctx *ctx, const Workspace &W, const mh_cmf_params *prm, mh_cmf_result *res,
-                float *crit_host, hipStream_t s);
+                float *crit_host, hipStream_t s, const HostResult *got = nullptr);
 }  // namespace
 
 MH_EXPORT int64_t mh_cmf_workspace_bytes(int64_t n)
@@ -1746,9 +1761,10 @@ MH_EXPORT int mh_cmf_solve(mh_ctx *ctx, float *u, const float *eigs, const float
     const Dims D{int(dims[0]), int(dims[1]), int(dims[2])};
 
     bool ran = false;
-    int rc = solve_onchip(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, &ran);
+    HostResult got;
+    int rc = solve_onchip(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, &got, &ran);
     if (rc) return rc;
-    if (ran) return read_result(ctx, W, prm, res, crit_host, s);
+    if (ran) return read_result(ctx, W, prm, res, crit_host, s, &got);
     Runner R(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s);
     R.may_slide = true;
     rc = R.init();
@@ -1777,18 +1793,26 @@ namespace {
 
 // Blocks; the criterion log, stop flag and iteration count of a solve.
 int read_result(mh_ctx *ctx, const Workspace &W, const mh_cmf_params *prm, mh_cmf_result *res,
-                float *crit_host, hipStream_t s)
+                float *crit_host, hipStream_t s, const HostResult *got)
 {
-    int ctrl[kCtrlWords];
-    MH_CHECK(ctx, hipMemcpyAsync(ctrl, W.ctrl, sizeof(ctrl), hipMemcpyDeviceToHost, s));
-    MH_CHECK(ctx, hipStreamSynchronize(s));
+    HostResult H;
+    if (!got) {
+        MH_CHECK(ctx, hipMemcpyAsync(&H, W.ctrl, H.bytes(prm), hipMemcpyDeviceToHost, s));
+        MH_CHECK(ctx, hipStreamSynchronize(s));
+        got = &H;
+    }
+    const int *ctrl = got->ctrl;
     if (ctrl[kStop] == mh::kSlideAborted) return kResumeSolve;
     const int ncrit = std::min(ctrl[kNcrit], kCritLogMax);
     float last = 0.f;
-    if (ncrit > 0)
+    if (ncrit > 0 && sizeof(int) * kCtrlWords + sizeof(float) * size_t(ncrit) <= H.bytes(prm)) {
+        last = got->crit[ncrit - 1];
+        if (crit_host) std::copy(got->crit, got->crit + ncrit, crit_host);
+    } else if (ncrit > 0) {
         MH_CHECK(ctx, hipMemcpy(&last, W.crit_log + ncrit - 1, sizeof(float), hipMemcpyDeviceToHost));
-    if (crit_host && ncrit > 0)
-        MH_CHECK(ctx, hipMemcpy(crit_host, W.crit_log, sizeof(float) * ncrit, hipMemcpyDeviceToHost));
+        if (crit_host)
+            MH_CHECK(ctx, hipMemcpy(crit_host, W.crit_log, sizeof(float) * ncrit, hipMemcpyDeviceToHost));
+    }
     if (res) {
         res->stopped = ctrl[kStop];
         res->ncrit = ncrit;
@@ -1957,9 +1981,10 @@ MH_EXPORT int mh_cmf_solve_noalloc(mh_ctx *ctx, float *u, const float *eigs, con
     hipStream_t s = (hipStream_t)stream;
     const Dims D{int(dims[0]), int(dims[1]), int(dims[2])};
     bool ran = false;
-    int rc = solve_onchip(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, &ran);
+    HostResult got;
+    int rc = solve_onchip(ctx, u, eigs, alpha, cs, ct, labels, D, n, prm, W, s, &got, &ran);
     if (rc) return rc;
-    if (ran) return read_result(ctx, W, prm, res, crit_host, s);
+    if (ran) return read_result(ctx, W, prm, res, crit_host, s, &got);
     // the method mh_cmf_solve tuned for these dims on this context, else the
     // untuned default; never tuned here (tuning creates events) and never
     // captured as a graph
