@@ -269,10 +269,11 @@ int mh_gvf(mh_ctx *ctx, float *g3_dev, float *swap3_dev, const float *v3_dev, co
            const int64_t dims[3], const mh_gvf_params *params, int iters, float *mag_dev,
            float *work_dev, void *stream);
 /* How mh_gvf runs its steps on this context (no counterpart in the
- * reference): 0 (default) two steps per launch, blocked along axis 0, for
- * volumes of 2^20 voxels or more; 1 one step per launch; 2 two per launch
- * whenever the volume allows. Results do not depend on it, bit for bit (the
- * magnitude sums of the checks may differ in their summation order). */
+ * reference): 0 (default) two to four steps per launch, blocked along axis 0,
+ * or one, as a cost model of the volume says (one up to about 80^3); 1 one step
+ * per launch; 2 several per launch whenever the volume allows. Results do not
+ * depend on it, bit for bit (the magnitude sums of the checks may differ in
+ * their summation order). */
 int mh_gvf_set_sweep(mh_ctx *ctx, int mode);
 
 /* Normalise non-zero vectors of g (SoA x3) to unit length

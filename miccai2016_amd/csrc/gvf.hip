@@ -1,6 +1,7 @@
 // Gradient vector flow on gfx950: explicit-Euler steps on the three SoA
 // components, ping-ponging two buffers, mirrored neighbours at the faces;
-// one step per launch, or two per launch in a sweep along axis 0.
+// one step per launch, or two to four per launch in a sweep along axis 0.
+#include "cmf_words.h"
 #include "mh_common.h"
 #include "mh_reduce.h"
 
@@ -74,147 +75,186 @@ gvf_step_kernel(float *__restrict__ out, const float *__restrict__ g, const floa
     if (threadIdx.x == 0) partials[blockIdx.x] = dmag;
 }
 
-// Two steps per launch, temporally blocked along axis 0 (as the max-flow
-// sweep is). A work-group owns an output tile of TY x TX voxels in the
-// (axis 1, axis 2) plane and a chunk of planes [z0, z1), one thread per point
-// of the tile widened by 2 on every side (E2). Step z loads g of plane z + 2
-// ahead of its use, puts g of plane z into LDS, and after the step's one
-// barrier computes
-//   level A: the first step at plane z on the tile widened by 1 (E1), from
-//            LDS (in-plane neighbours) and registers (planes z - 1, z + 1),
-//            into LDS by plane parity;
-//   level B: the second step at plane z - 1 on the tile, from the level-A
-//            results of the previous step in LDS (written before this
-//            step's barrier) and in registers (planes z - 2, z - 1, z),
-//            and stores it.
-// LDS holds two planes of each (by plane parity), so one barrier per step
-// orders every write before the reads that need it and after the reads of
-// the plane two steps back. The per-voxel arithmetic is gvf_voxel's, so the
-// result equals two launches of gvf_step_kernel bit for bit. With
-// `partials`, each work-group stores the sum of |delta| of its second step.
-template <int TY, int TX, int NT>
+// word 3 of a buffer's resource: a 32-bit format, offsets checked against its
+// bytes (loads beyond it give zero, stores none)
+constexpr int kRawBuffer = 0x00027000;
+
+// L steps per launch, temporally blocked along axis 0 (as the max-flow sweep
+// is). A work-group owns an output tile of TY x TX voxels in the (axis 1, axis 2)
+// plane and a chunk of planes [z0, z1), one thread per point of the tile widened
+// by L on every side. Step z puts g of plane z into LDS and after the step's one
+// barrier computes, for l = 1 .. L,
+//   level l: the l-th step at plane z - l + 1 on the tile widened by L - l, from
+//            level l - 1 of the same plane in LDS (written a step ago; level 0:
+//            before the barrier) and of the planes around it in registers,
+//            into LDS by plane parity; level L is stored.
+// LDS holds two planes of each level (by plane parity), so one barrier per step
+// orders every write before the reads that need it and after the reads of the
+// plane two steps back. The per-voxel arithmetic is gvf_voxel's, so the result
+// equals L launches of gvf_step_kernel bit for bit. With `partials`, each
+// work-group stores the sum of |delta| of its last step.
+//
+// Loads run two planes ahead and go through buffer resources, whose bounds mask
+// the lanes outside the volume: without branches around them the compiler knows
+// how many are under way and waits for none but the plane it needs. They are
+// issued between the levels (all seven at once hold up the waves at the step's
+// start: 14.3 against 13.2 us per GVF step at 150 x 128 x 141). A step of all
+// work-groups takes about 1.0 + 0.25 L us, the first part for the loads and
+// stores of 64 threads each (tiles of 24 columns 1.2: rows of 128 bytes off
+// their alignment), the second for the arithmetic; so three and four levels in
+// wide tiles win although their halos cost more. Two levels with the loads one
+// plane ahead, which this replaces: 16.7 us; one step per launch: 17.3.
+template <int TY, int TX, int NT, int L>
 __global__ void __launch_bounds__(NT)
 gvf_sweep_kernel(float *__restrict__ out, const float *__restrict__ g, const float *__restrict__ v,
                  const float *__restrict__ r, int d0, int d1, int d2, float mu, float dt, float rss0,
                  float rss1, float rss2, int zchunk, float *__restrict__ partials)
 {
-    constexpr int EY = TY + 4, EX = TX + 4, NE = EY * EX;
+    constexpr int EY = TY + 2 * L, EX = TX + 2 * L, NE = EY * EX;
     static_assert(NE <= NT, "one point per thread");
-    __shared__ float sG[2][3][NE];  // g of plane z, by plane parity
-    __shared__ float sH[2][3][NE];  // level-A result of plane z, by plane parity
+    extern __shared__ float lds[];  // level l of plane parity q, component c: 3 (2 l + q) + c
     const unsigned b = mh::xcd_block(blockIdx.x, gridDim.x);
     const int ntx = (d2 + TX - 1) / TX, nty = (d1 + TY - 1) / TY;
     const int tx = int(b % unsigned(ntx)), ty = int((b / unsigned(ntx)) % unsigned(nty));
     const int tz = int(b / unsigned(ntx * nty));
-    const int x0 = tx * TX, y0 = ty * TY, z0 = tz * zchunk;
-    const int z1 = min(z0 + zchunk, d0);
+    const int z0 = tz * zchunk, z1 = min(z0 + zchunk, d0);
     const int t = int(threadIdx.x);
     const bool live = t < NE;
     const int yy = live ? t / EX : 0, xx = live ? t % EX : 0;
     const int p = yy * EX + xx;
-    const int y = y0 - 2 + yy, x = x0 - 2 + xx;
+    const int y = ty * TY - L + yy, x = tx * TX - L + xx;
     const bool inv = live && y >= 0 && y < d1 && x >= 0 && x < d2;
-    const bool inE1 = inv && yy >= 1 && yy <= TY + 2 && xx >= 1 && xx <= TX + 2;
-    const bool inO = inv && yy >= 2 && yy <= TY + 1 && xx >= 2 && xx <= TX + 1;
-    // in-plane neighbours in LDS, mirrored at the faces (inside E2 for E1)
+    // levels up to this one are computed at this point
+    const int most = inv ? min(min(min(yy, EY - 1 - yy), min(xx, EX - 1 - xx)), L) : 0;
+    // in-plane neighbours in LDS, mirrored at the faces
     const int pym = y > 0 ? p - EX : p + EX, pyp = y < d1 - 1 ? p + EX : p - EX;
     const int pxm = x > 0 ? p - 1 : p + 1, pxp = x < d2 - 1 ? p + 1 : p - 1;
-    const int64_t n = int64_t(d0) * d1 * d2, st0 = int64_t(d1) * d2;
-    const int64_t ip = inv ? int64_t(y) * d2 + x : 0;
-    auto at = [&](int z) { return int64_t(z) * st0 + ip; };
+    const int64_t n = int64_t(d0) * d1 * d2;
+    const unsigned st0 = unsigned(d1) * unsigned(d2), plane = 4u * st0;
+    // byte offset in a plane; lanes that load or store nothing lie beyond it
+    const unsigned here4 = 4u * (unsigned(y) * unsigned(d2) + unsigned(x));
+    const unsigned in_g = inv ? here4 : ~0u, in_v = most > 0 ? here4 : ~0u, in_o = most == L ? here4 : ~0u;
+    auto load = [&](const float *f, int k, unsigned off) {
+        return __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(
+                       __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(f) + int64_t(k) * st0, 0,
+                                                         int(plane), kRawBuffer),
+                       int(off), 0, 0));
+    };
 
-    const int zs = max(z0 - 1, 0);  // first level-A plane
-    const int zend = z1;            // last step (level A only below d0)
-    float gm[3], gc[3], gp[3], gn[3];    // g at planes z - 1, z, z + 1 (mirrored), z + 2
-    float vA[3], vB[3], vN[3];           // v at planes z, z - 1, z + 1
-    float rA = 0.f, rB = 0.f, rN = 0.f;
-    float h2[3], h1[3], h0[3];           // level A at planes z - 2, z - 1, z
+    const int zs = max(z0 - (L - 1), 0);   // first plane of level 1
+    const int zend = z1 - 1 + (L - 1);     // the last step
+    // Planes in registers, by their distance from zs modulo 6 (g, v, r) or 3 (the
+    // levels), so that none is ever moved: a move would wait for the loads.
+    float G[6][3], V[6][3], R[6], H[L][3][3];  // H[0] is not used
     float dsum = 0.f;
 #pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        R[k] = 0.f;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) G[k][c] = V[k][c] = 0.f;
+    }
+#pragma unroll
+    for (int l = 0; l < L; ++l)
+#pragma unroll
+        for (int k = 0; k < 9; ++k) H[l][k / 3][k % 3] = 0.f;
+    // inputs that step z is the first to use, loaded two steps ahead: g of plane
+    // z + 1, v and r of plane z (beyond the volume: the last plane's, not used)
+    auto fetch_g = [&](auto PH, int z) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) G[(PH + 1) % 6][c] = load(g + c * n, min(z + 1, d0 - 1), in_g);
+    };
+    auto fetch_v = [&](auto PH, int z) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) V[PH][c] = load(v + c * n, min(z, d0 - 1), in_v);
+        R[PH] = load(r, min(z, d0 - 1), in_v);
+    };
+#pragma unroll
     for (int c = 0; c < 3; ++c) {
-        gm[c] = gc[c] = gp[c] = gn[c] = vA[c] = vB[c] = vN[c] = h2[c] = h1[c] = h0[c] = 0.f;
+        G[0][c] = load(g + c * n, zs, in_g);
+        G[5][c] = load(g + c * n, max(zs - 1, 0), in_g);
     }
-    if (inv) {
-        const int zm = zs > 0 ? zs - 1 : zs + 1, zp = zs < d0 - 1 ? zs + 1 : zs - 1;
+    fetch_g(std::integral_constant<int, 0>{}, zs);
+    fetch_v(std::integral_constant<int, 0>{}, zs);
+    fetch_g(std::integral_constant<int, 1>{}, zs + 1);
+    fetch_v(std::integral_constant<int, 1>{}, zs + 1);
+    auto step = [&](auto PH, int z) {
+        if (live) {
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            gc[c] = g[c * n + at(zs)];
-            gm[c] = g[c * n + at(zm)];
-            gp[c] = g[c * n + at(zp)];
+            for (int c = 0; c < 3; ++c) lds[(3 * (PH % 2) + c) * NE + p] = G[PH][c];
         }
-    }
-    if (inE1) {
+        mh::lds_barrier();
+        mh::unrolled_while<L>([&](auto LC) {
+            constexpr int l = LC + 1, kk = (PH + 13 - l) % 6;  // its plane: z - l + 1
+            constexpr int q = kk % 2;
+            const int k = z - l + 1;
+            float o[3] = {0.f, 0.f, 0.f};
+            const bool on = k >= z0 - (L - l) && k >= 0 && k < z1 + (L - l) && k < d0;
+            if (on) {
+                float(&mid)[3] = l == 1 ? G[kk] : H[l - 1][kk % 3];
+                float(&below)[3] = l == 1 ? G[(kk + 5) % 6] : H[l - 1][(kk + 2) % 3];
+                float(&above)[3] = l == 1 ? G[(kk + 1) % 6] : H[l - 1][(kk + 1) % 3];
+                if (k == 0) {  // mirrored
 #pragma unroll
-        for (int c = 0; c < 3; ++c) vA[c] = v[c * n + at(zs)];
-        rA = r[at(zs)];
-    }
-    for (int z = zs; z <= zend; ++z) {
-        const bool la = z < d0;                  // level A at plane z
-        const bool lb = z - 1 >= z0;             // level B at plane z - 1 (< z1 since z <= z1)
-        const int q = z & 1, qb = (z - 1) & 1;
-        // inputs of the next step
-        if (inv && z + 1 < d0) {
-            if (z + 2 < d0) {
+                    for (int c = 0; c < 3; ++c) below[c] = above[c];
+                }
+                if (k == d0 - 1) {
 #pragma unroll
-                for (int c = 0; c < 3; ++c) gn[c] = g[c * n + at(z + 2)];
-            } else {  // plane z + 1 is the last: its upper neighbour mirrors to plane z
+                    for (int c = 0; c < 3; ++c) above[c] = below[c];
+                }
+                if (most >= l) {
+                    const float *S = lds + 3 * (2 * (l - 1) + q) * NE;
+                    float dl[3];
 #pragma unroll
-                for (int c = 0; c < 3; ++c) gn[c] = gc[c];
+                    for (int c = 0; c < 3; ++c) {
+                        dl[c] = gvf_voxel(mid[c], below[c], above[c], S[c * NE + pym], S[c * NE + pyp],
+                                          S[c * NE + pxm], S[c * NE + pxp], V[kk][c], R[kk], mu, dt,
+                                          rss0, rss1, rss2, o[c]);
+                        if (l < L) lds[(3 * (2 * l + q) + c) * NE + p] = o[c];
+                    }
+                    if (l == L && partials) dsum += gvf_mag(dl[0], dl[1], dl[2]);
+                }
             }
-        }
-        if (inE1 && z + 1 < d0) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) vN[c] = v[c * n + at(z + 1)];
-            rN = r[at(z + 1)];
-        }
-        if (la && live) {
-#pragma unroll
-            for (int c = 0; c < 3; ++c) sG[q][c][p] = gc[c];
-        }
-        __syncthreads();
-        if (la && inE1) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                h0[c] = 0.f;
-                (void)gvf_voxel(gc[c], gm[c], gp[c], sG[q][c][pym], sG[q][c][pyp], sG[q][c][pxm],
-                                sG[q][c][pxp], vA[c], rA, mu, dt, rss0, rss1, rss2, h0[c]);
-                sH[q][c][p] = h0[c];
+                if (l < L)
+                    H[l < L ? l : 0][kk % 3][c] = o[c];
+                else
+                    __builtin_amdgcn_raw_buffer_store_b32(
+                        __builtin_bit_cast(unsigned, o[c]),
+                        __builtin_amdgcn_make_buffer_rsrc(out + c * n + int64_t(on ? k : 0) * st0, 0,
+                                                          on ? int(plane) : 0, kRawBuffer),
+                        int(in_o), 0, 0);
             }
-        }
-        if (lb && inO) {
-            const int zb = z - 1;
-            float dl[3];
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const float below = zb > 0 ? h2[c] : h0[c];
-                const float above = zb < d0 - 1 ? h0[c] : h2[c];
-                float o;
-                dl[c] = gvf_voxel(h1[c], below, above, sH[qb][c][pym], sH[qb][c][pyp],
-                                  sH[qb][c][pxm], sH[qb][c][pxp], vB[c], rB, mu, dt, rss0, rss1,
-                                  rss2, o);
-                out[c * n + at(zb)] = o;
-            }
-            if (partials) dsum += gvf_mag(dl[0], dl[1], dl[2]);
-        }
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            gm[c] = gc[c];
-            gc[c] = gp[c];
-            gp[c] = gn[c];
-            h2[c] = h1[c];
-            h1[c] = h0[c];
-            vB[c] = vA[c];
-            vA[c] = vN[c];
-        }
-        rB = rA;
-        rA = rN;
-    }
+            __builtin_amdgcn_sched_barrier(0);
+            if (l == 1) fetch_g(std::integral_constant<int, (PH + 2) % 6>{}, z + 2);
+            if (l == 2) fetch_v(std::integral_constant<int, (PH + 2) % 6>{}, z + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            return true;
+        });
+    };
+    for (int z = zs; z <= zend; z += 6)
+        mh::unrolled_while<6>([&](auto PH) {
+            step(PH, z + PH);
+            return z + PH < zend;
+        });
     if (!partials) return;
     dsum = mh::block_reduce<SumOp>(dsum);
-    if (threadIdx.x == 0) partials[blockIdx.x] = dsum;
+    if (t == 0) partials[blockIdx.x] = dsum;
 }
 
-constexpr int kGvfTY = 11, kGvfTX = 64, kGvfNT = 1024;
+struct GvfShape {
+    int ty, tx, nt, levels;
+    double unit;  // microseconds a plane step of all resident work-groups takes
+    const void *kernel;
+    int lds() const { return 4 * levels * 6 * (ty + 2 * levels) * (tx + 2 * levels); }
+};
+#define GVF_SHAPE(TY, TX, NT, L, UNIT) \
+    {TY, TX, NT, L, UNIT, reinterpret_cast<const void *>(&gvf_sweep_kernel<TY, TX, NT, L>)}
+const GvfShape kGvfShapes[] = {GVF_SHAPE(15, 48, 1024, 2, 1.6), GVF_SHAPE(12, 50, 1024, 3, 1.6),
+                               GVF_SHAPE(10, 58, 1024, 3, 1.52), GVF_SHAPE(6, 74, 960, 3, 1.34),
+                               GVF_SHAPE(24, 24, 1024, 4, 1.95)};
+#undef GVF_SHAPE
 
 // Sum of the per-block partials in block order (one work-group).
 __global__ void __launch_bounds__(mh::kBlock)
@@ -267,34 +307,46 @@ MH_EXPORT int mh_gvf_response(mh_ctx *ctx, float *r, const float *v3, int64_t n,
     return MH_OK;
 }
 
-// Plane chunk of the two-step kernel from the launch cost model of the
-// max-flow sweep: work-groups run in ceil(groups / slots) waves of about
-// (chunk + 2) plane steps; the chunk must leave at most max_groups groups.
-int gvf_zchunk(mh_ctx *ctx, const int64_t dims[3], int64_t max_groups)
+struct GvfPlan {
+    const GvfShape *shape = nullptr;  // null: one step per launch
+    int zchunk = 0;
+    int64_t groups = 0;
+};
+
+// The shape and plane chunk that take the fewest microseconds per step: a
+// launch's work-groups run in ceil(groups / slots) waves of chunk + 2 (levels - 1)
+// plane steps, and a launch costs 2.5 beside them; the chunk must leave at most
+// max_groups groups. One step per launch takes 2.2 + 5.6 per million voxels, the
+// less up to about 80^3 (5.2 us a step there, 5.5 in three levels; 96^3 7.2 and
+// 5.8, 120^3 11.9 and 8.7, 220 x 215 x 210 94 and 41). `any`: a sweep in any case.
+GvfPlan gvf_plan(mh_ctx *ctx, const int64_t dims[3], int iters, int64_t max_groups, bool any)
 {
-    int cus = 0, per = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess)
-        cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per, reinterpret_cast<const void *>(&gvf_sweep_kernel<kGvfTY, kGvfTX, kGvfNT>), kGvfNT,
-            0) != hipSuccess)
-        per = 0;
-    (void)hipGetLastError();
-    const int64_t slots = (cus > 0 && per > 0) ? int64_t(cus) * per : 256;
-    const int64_t tiles = ((dims[2] + kGvfTX - 1) / kGvfTX) * ((dims[1] + kGvfTY - 1) / kGvfTY);
+    GvfPlan best;
+    if (4 * dims[1] * dims[2] >= (int64_t(1) << 31)) return best;  // bytes of a buffer resource
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
+        cus <= 0)
+        cus = 256;
+    double cost = any ? 1e30 : 2.2 + 5.6e-6 * double(dims[0]) * double(dims[1]) * double(dims[2]);
     const int d0 = int(dims[0]);
-    int best = 0;
-    int64_t best_cost = -1;
-    for (int z = 1; z <= d0; ++z) {
-        const int64_t groups = tiles * ((d0 + z - 1) / z);
-        if (groups > max_groups) continue;
-        const int64_t cost = ((groups + slots - 1) / slots) * (z + 2);
-        if (best_cost < 0 || cost < best_cost || (cost == best_cost && z > best)) {
-            best_cost = cost;
-            best = z;
+    for (const GvfShape &S : kGvfShapes) {
+        if (iters < S.levels) continue;
+        const int64_t tiles = ((dims[2] + S.tx - 1) / S.tx) * ((dims[1] + S.ty - 1) / S.ty);
+        for (int z = 1; z <= d0; ++z) {
+            const int64_t groups = tiles * ((d0 + z - 1) / z);
+            if (groups > max_groups) continue;
+            const double c = (double((groups + cus - 1) / cus) * (z + 2 * (S.levels - 1)) * S.unit + 2.5) /
+                             S.levels;
+            if (c < cost) {
+                cost = c;
+                best.shape = &S;
+                best.zchunk = z;
+                best.groups = groups;
+            }
         }
     }
-    return best;  // 0: none fits
+    (void)hipGetLastError();
+    return best;
 }
 
 MH_EXPORT int mh_gvf(mh_ctx *ctx, float *g3, float *swap3, const float *v3, const float *r,
@@ -309,15 +361,15 @@ MH_EXPORT int mh_gvf(mh_ctx *ctx, float *g3, float *swap3, const float *v3, cons
     const unsigned nb = mh::blocks_for(n);
     hipStream_t s = (hipStream_t)stream;
     float *src = g3, *dst = swap3;
-    // two steps per launch where the volume fills the device with them
-    // (automatic: from 2^20 voxels on); the partial sums of the last launch
-    // fit in the workspace's nb floats
-    int zc = 0;
-    if (ctx->gvf_sweep != 1 && iters >= 2 && (ctx->gvf_sweep == 2 || n >= (int64_t(1) << 20)))
-        zc = gvf_zchunk(ctx, dims, int64_t(nb));
-    const int64_t groups = zc ? ((dims[2] + kGvfTX - 1) / kGvfTX) * ((dims[1] + kGvfTY - 1) / kGvfTY) *
-                                    ((dims[0] + zc - 1) / zc)
-                              : 0;
+    // several steps per launch where that is faster; the partial sums of the
+    // last launch fit in the workspace's nb floats
+    GvfPlan P;
+    if (ctx->gvf_sweep != 1 && iters >= 2)
+        P = gvf_plan(ctx, dims, iters, int64_t(nb), ctx->gvf_sweep == 2);
+    const int levels = P.shape ? P.shape->levels : 1;
+    if (P.shape)
+        MH_CHECK(ctx, hipFuncSetAttribute(P.shape->kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          P.shape->lds()));
     int it = 0;
     auto step = [&](float *parts) {
         hipLaunchKernelGGL(gvf_step_kernel, dim3(nb), dim3(mh::kBlock), 0, s, dst, src, v3, r,
@@ -330,19 +382,21 @@ MH_EXPORT int mh_gvf(mh_ctx *ctx, float *g3, float *swap3, const float *v3, cons
         dst = t;
         ++it;
     };
-    if (zc && iters % 2 == 1) step((mag && iters == 1) ? work : nullptr);  // an odd first step
-    while (zc && it + 2 <= iters) {
-        float *parts = (mag && it + 2 == iters) ? work : nullptr;
-        hipLaunchKernelGGL((gvf_sweep_kernel<kGvfTY, kGvfTX, kGvfNT>), dim3(unsigned(groups)),
-                           dim3(kGvfNT), 0, s, dst, src, v3, r, int(dims[0]), int(dims[1]),
-                           int(dims[2]), p->mu, p->dt, p->rss[0], p->rss[1], p->rss[2], zc, parts);
+    while ((iters - it) % levels) step((mag && it == iters - 1) ? work : nullptr);
+    while (P.shape && it < iters) {
+        float *parts = (mag && it + levels == iters) ? work : nullptr;
+        int d0 = int(dims[0]), d1 = int(dims[1]), d2 = int(dims[2]);
+        float mu = p->mu, dt = p->dt, r0 = p->rss[0], r1 = p->rss[1], r2 = p->rss[2];
+        void *args[] = {&dst, &src, &v3, &r, &d0, &d1, &d2, &mu, &dt, &r0, &r1, &r2, &P.zchunk, &parts};
+        MH_CHECK(ctx, hipLaunchKernel(P.shape->kernel, dim3(unsigned(P.groups)),
+                                      dim3(unsigned(P.shape->nt)), args, size_t(P.shape->lds()), s));
         if (parts)
             hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(mh::kBlock), 0, s, parts,
-                               int(groups), mag);
+                               int(P.groups), mag);
         float *t = src;
         src = dst;
         dst = t;
-        it += 2;
+        it += levels;
     }
     while (it < iters) step((mag && it == iters - 1) ? work : nullptr);
     MH_CHECK_LAUNCH(ctx, "gvf kernels");
