@@ -405,8 +405,41 @@ __constant__ float kSorter[6][4] = {
 
 __device__ __forceinline__ void atomic_max_nonneg(float *addr, float v)
 {
-    // non-negative floats order like their bit patterns
-    atomicMax(reinterpret_cast<unsigned *>(addr), __float_as_uint(v));
+    // Non-negative floats order like their bit patterns. The maximum only grows,
+    // so what is not above a value seen there needs no atomic: one per
+    // work-group on one address, at 12 ns each, took the 149 us of eig_kernel at
+    // 160 x 131 x 150 (12281 work-groups), now 76.
+    unsigned *a = reinterpret_cast<unsigned *>(addr);
+    if (__float_as_uint(v) > __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(a, __float_as_uint(v));
+}
+
+// Six consecutive floats of a voxel, in pairs where the array is aligned to them
+// (every 24th byte then is): half as many accesses of 24-byte strides.
+__device__ __forceinline__ void load6(const float *p, float (&v)[6])
+{
+    if ((reinterpret_cast<uintptr_t>(p) & 7) == 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float2 w = reinterpret_cast<const float2 *>(p)[k];
+            v[2 * k] = w.x;
+            v[2 * k + 1] = w.y;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) v[k] = p[k];
+    }
+}
+__device__ __forceinline__ void store6(float *p, const float (&v)[6])
+{
+    if ((reinterpret_cast<uintptr_t>(p) & 7) == 0) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            reinterpret_cast<float2 *>(p)[k] = make_float2(v[2 * k], v[2 * k + 1]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) p[k] = v[k];
+    }
 }
 
 struct MaxNonNeg {
@@ -426,7 +459,8 @@ eig_kernel(const float *in6, float *out6, int64_t n, int maxiter, float *norm_ma
     const int64_t i = int64_t(b) * blockDim.x + threadIdx.x;
     float nrm = 0.f;
     if (i < n) {
-        const float *h = in6 + 6 * i;
+        float h[6];
+        load6(in6 + 6 * i, h);
         float d[3] = {h[0], h[1], h[2]};
         float o[3] = {h[5], h[4], h[3]};  // o[r]: element (p, q), r = 3 - p - q
         float qv[3] = {0.f, 0.f, 0.f};
@@ -500,8 +534,7 @@ eig_kernel(const float *in6, float *out6, int64_t n, int maxiter, float *norm_ma
         } else {
             for (int k = 0; k < 6; ++k) res[k] = __builtin_nanf("");
         }
-        float *e = out6 + 6 * i;
-        for (int k = 0; k < 6; ++k) e[k] = res[k];
+        store6(out6 + 6 * i, res);
     }
     if (norm_max) {
         nrm = mh::block_reduce<MaxNonNeg>(nrm);
@@ -533,7 +566,8 @@ vesselness_kernel(float *__restrict__ val, float *__restrict__ quat, const float
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float c = c_value >= 0.f ? c_value : 0.5f * (*norm_max);
-    const float *e = e6 + 6 * i;
+    float e[6];
+    load6(e6 + 6 * i, e);
     const float l1 = fabsf(e[0]);
     float l2 = bright ? e[1] : -e[1];
     float l3 = bright ? e[2] : -e[2];
