@@ -63,6 +63,14 @@ TRAFFIC_SWEEP_PAIR_PER_VOXEL_ITER = {1: 38.8, 7: 30.2}
 PAIR_TILES = (1, 4, 5, 6, 7)
 # iterations per pass of each tile shape (1-based)
 SWEEP_LEVELS = {1: 2, 2: 2, 3: 2, 4: 2, 5: 2, 6: 3, 7: 3, 8: 4, 9: 4}
+# Solves that stay on the chip (volumes of up to 2^21 voxels, the automatic method):
+# vector instructions per voxel-iteration of the p- and the u-step with eigenvalues
+# (l0, l1, l1), and the rate 256 compute units issue them at (64 lanes, 2.4 GHz);
+# bytes per voxel and solve: u0, alpha, cs, ct and the frame in, u out
+ONCHIP_VOXELS = 1 << 21
+ONCHIP_INSTRUCTIONS = 74.0
+VECTOR_ISSUE_T = 39.3
+ONCHIP_BYTES_PER_VOXEL = 32.0
 GRID_GROUP = 4                         # solves per group of the batched per-iteration kernels
 
 PARTS = ("grid", "plain", "plain64", "plain256", "ragged", "serve", "cpu", "sigmas")
@@ -301,7 +309,23 @@ def main():
             tile = args.sweep_tile or 1      # forced, not tuned
         step_s = secs / args.steps
         effective = value * BYTES_PER_VOXEL_ITER / 1e9
-        if tile:
+        if args.sweep == 0 and args.batched_sweep == 0 and n <= ONCHIP_VOXELS:
+            # solve after solve in the registers of one launch (the first two
+            # through the sweep where the pair tuner still had to time it)
+            achieved = value * ONCHIP_INSTRUCTIONS / 1e12
+            line["roofline"] = {
+                "bound": "vector issue", "achieved": achieved, "peak": VECTOR_ISSUE_T,
+                "unit": "T lane-instructions/s", "frac": achieved / VECTOR_ISSUE_T,
+                "traffic": ONCHIP_BYTES_PER_VOXEL * n * S,
+                "kernel": f"cmf_onchip_kernel: one launch = {S} solves of {args.iters} max-flow "
+                          "iterations, the state in registers, brick faces as tagged words",
+                "algorithmic": f"{ONCHIP_INSTRUCTIONS:.0f} vector instructions per "
+                               "voxel-iteration (p-step 47, u-step 27)",
+                "us_per_iteration": step_s / (S * args.iters) * 1e6,
+                "algorithmic_hbm_GBs": ONCHIP_BYTES_PER_VOXEL * n * S / step_s / 1e9,
+                "effective_GBs_84B": effective,
+                "effective_frac_84B": effective / HBM_PEAK_GBS}
+        elif tile:
             # the groups ran one after another through the multi-level sweep:
             # one launch is one pass of up to L iterations over a pair of
             # solves (the 1024-thread tile shapes of up to three levels) or
