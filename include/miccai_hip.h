@@ -412,6 +412,17 @@ int mh_cmf_sweep_choice(mh_ctx *ctx, const int64_t dims[3], int *tile, int *zchu
  * for them (the batched solver then uses the single-solve choice). */
 int mh_cmf_batched_sweep_choice(mh_ctx *ctx, const int64_t dims[3], int *tile, int *zchunk);
 
+/* Packed volumes of a ragged batch (as mh_cmf_solve_ragged takes them) that share
+ * a launch on the chip: eigenvalues (l0, l1, l1), two to eight volumes whose
+ * work-groups fit the device together. solved_host[v] becomes 1 and res[v] is set
+ * for those, 0 for the others, which are as they were and left to the other
+ * solvers; results do not depend on it, bit for bit. work_dev: 64 MiB. Blocks. */
+#define MH_CMF_RAGGED_ONCHIP_BYTES (64ll << 20)
+int mh_cmf_ragged_onchip(mh_ctx *ctx, float *u_dev, const float *eigs_dev, const float *alpha_dev,
+                         const float *cs_dev, const float *ct_dev, int nvol, const int64_t *vdims_host,
+                         const int64_t *voff_host, const mh_cmf_params *params, void *work_dev,
+                         int64_t work_bytes, mh_cmf_result *res, int *solved_host, void *stream);
+
 /* Packed ragged batch: volume v has dims vdims_host[3v..3v+2] and its fields
  * start at element offset voff_host[v] in every packed array (u, eigs*3,
  * alpha, cs, ct). No counterpart in the reference. Blocks. */

@@ -123,7 +123,10 @@ SIGNATURES = {
     "mh_cmf_ragged_workspace_bytes": (i64, [i64, i32]),
     "mh_cmf_solve_ragged": (i32, [vp, vp, vp, vp, vp, vp, i32, vp, vp, C.POINTER(CmfParams), vp,
                                   i64, C.POINTER(CmfResult), vp]),
+    "mh_cmf_ragged_onchip": (i32, [vp, vp, vp, vp, vp, vp, i32, vp, vp, C.POINTER(CmfParams), vp,
+                                   i64, C.POINTER(CmfResult), vp, vp]),
 }
+CMF_RAGGED_ONCHIP_BYTES = 64 << 20
 
 
 def lib():

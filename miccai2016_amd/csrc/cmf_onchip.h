@@ -48,4 +48,23 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &plan, const OnchipSolve *solves, i
                int64_t work_bytes, hipStream_t s, bool *ran,
                std::vector<int> *finished = nullptr, void *head = nullptr, size_t head_bytes = 0);
 
+// Solves of several volumes side by side, eigenvalues (l0, l1, l1), no seeds: the
+// plan that takes the least of the device for one of them (v = 0: none), and the
+// launch of up to 8 whose plans' work-groups fit the device together.
+constexpr size_t kOnchipMany = 8;
+struct OnchipVolume {
+    OnchipPlan plan;
+    OnchipSolve solve;
+    OnchipFields F;
+    int dims[3];
+    int64_t head_bytes;  // of its control words and criteria
+};
+OnchipPlan onchip_plan_many(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm);
+// Enqueue and wait. `heads` (device) holds the volumes' control words and criteria
+// one after another and comes to `host`. `ran`: every volume has its result, else
+// every u is as it was.
+int onchip_run_many(mh_ctx *ctx, const OnchipVolume *vols, int nvol, const mh_cmf_params *prm,
+                    void *work, int64_t work_bytes, void *heads, hipStream_t s, std::vector<char> *host,
+                    bool *ran);
+
 }  // namespace mh

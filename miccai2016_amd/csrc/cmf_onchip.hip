@@ -74,6 +74,18 @@ struct Args {
     int *abort;
 };
 
+// One volume's solves, or one solve of each of up to N volumes side by side:
+// volume v's work-groups are first[v] .. first[v + 1] - 1. An iteration's two
+// exchanges take as long for a small volume as for a large one (64^3 2.6 us on
+// 128 or 256 compute units), so several share them (packed per-iteration
+// kernels: 10.6 us an iteration for a few volumes below 80^3).
+template <int N>
+struct ArgsOf {
+    Args a[N];
+    int n, first[N + 1];
+};
+constexpr int kMany = int(mh::kOnchipMany);
+
 // Where a thread's 128 registers do not hold its planes, cs and ct are in LDS:
 // of 8 planes all cs and the upper four's ct (160 KB are then full), of 4 planes
 // with pointwise eigenvalues all of both.
@@ -84,10 +96,18 @@ constexpr int lds_bytes(int v, int mode)
                 (caps_in_lds(v, mode) ? (v + 4) * kMaxThreads : 0));
 }
 
-template <int V, int MODE, bool SUP, bool DEFER>
+template <int V, int MODE, bool SUP, bool DEFER, int N = 1>
 __global__ void __launch_bounds__(kMaxThreads)
-cmf_onchip_kernel(const Args A)
+cmf_onchip_kernel(const ArgsOf<N> L)
 {
+    unsigned b = mh::xcd_block(blockIdx.x, gridDim.x);
+    int vol = 0;
+    if (N > 1) {
+        while (vol + 1 < L.n && int(b) >= L.first[vol + 1]) ++vol;
+        vol = __builtin_amdgcn_readfirstlane(vol);
+        b -= unsigned(L.first[vol]);
+    }
+    const Args &A = L.a[vol];
     constexpr int G = V < 4 ? V : 4, NG = V / G;
     constexpr int NF = MODE == kAxial ? 3 : MODE == kConst ? 4 : 7;
     constexpr int kTile = NG * kCells;  // LDS vectors of one field
@@ -106,7 +126,6 @@ cmf_onchip_kernel(const Args A)
     int *fail = reinterpret_cast<int *>(red + kRedFloats - 1);
 
     const int per = A.nt1 * A.nt2 * A.nz;
-    const unsigned b = mh::xcd_block(blockIdx.x, gridDim.x);
     const int slot = int(b) / per, lb = int(b) - slot * per;
     const int bx = lb % A.nt2, by = (lb / A.nt2) % A.nt1, bz = lb / (A.nt1 * A.nt2);
     const bool live = t < nc;
@@ -631,7 +650,150 @@ int64_t nwords_of(const OnchipPlan &P, int slots)
 {
     return int64_t(slots) * P.blocks() * (2 * (P.b1 * P.b2 + words_of(P)) + 2);
 }
+Args args_of(const OnchipPlan &P, const OnchipFields &F, const int dims[3], const mh_cmf_params *prm)
+{
+    Args A{};
+    A.F = F;
+    A.d0 = dims[0];
+    A.d1 = dims[1];
+    A.d2 = dims[2];
+    A.b1 = P.b1;
+    A.b2 = P.b2;
+    A.nt1 = P.nt1;
+    A.nt2 = P.nt2;
+    A.nz = P.nz;
+    A.num_iter = prm->num_iter;
+    A.update = prm->update;
+    A.rcc = prm->rcc;
+    A.inv_rcc = float(1.0 / double(prm->rcc));
+    A.rs0 = prm->rs[0];
+    A.rs1 = prm->rs[1];
+    A.rs2 = prm->rs[2];
+    A.ss0 = prm->ss[0];
+    A.ss1 = prm->ss[1];
+    A.ss2 = prm->ss[2];
+    A.error_bound = prm->error_bound;
+    A.inv_n_rcc = float(1.0 / (double(int64_t(dims[0]) * dims[1] * dims[2]) * double(prm->rcc)));
+    A.sq0 = prm->sqev[0];
+    A.sq1 = prm->sqev[1];
+    A.sq2 = prm->sqev[2];
+    A.rq0 = float(1.0 / double(prm->sqev[0]));
+    A.rq1 = float(1.0 / double(prm->sqev[1]));
+    A.rq2 = float(1.0 / double(prm->sqev[2]));
+    A.A = axi_params(prm);
+    return A;
+}
 }  // namespace
+
+OnchipPlan onchip_plan_many(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm)
+{
+    OnchipPlan best;
+    const int cus = ctx->device < kMaxDevices ? compute_units(ctx) : 0;
+    double best_cost = 0;
+    if (mode_of(prm) != kAxial) return best;
+    for (int n2 = 1; n2 <= std::min(dims[2], 16); ++n2) {
+        const int b2 = (dims[2] + n2 - 1) / n2;
+        if (b2 > kMaxThreads) continue;
+        const int least = (dims[1] + kMaxThreads / b2 - 1) / (kMaxThreads / b2);
+        for (int n1 = least; n1 <= std::min(dims[1], least + 4); ++n1) {
+            OnchipPlan P;
+            P.v = kMaxPlanes;
+            P.b1 = (dims[1] + n1 - 1) / n1;
+            P.b2 = b2;
+            P.nt1 = (dims[1] + P.b1 - 1) / P.b1;
+            P.nt2 = (dims[2] + b2 - 1) / b2;
+            P.nz = (dims[0] + P.v - 1) / P.v;
+            const double cost = iteration_us(P) * P.blocks();
+            if (P.blocks() <= cus && plan_fits(P) && (best.v == 0 || cost < best_cost)) {
+                best = P;
+                best_cost = cost;
+            }
+        }
+    }
+    return best;
+}
+
+int onchip_run_many(mh_ctx *ctx, const OnchipVolume *vols, int nvol, const mh_cmf_params *prm,
+                    void *work, int64_t work_bytes, void *heads, hipStream_t s, std::vector<char> *host,
+                    bool *ran)
+{
+    *ran = false;
+    const int cus = compute_units(ctx);
+    ArgsOf<kMany> L{};
+    int64_t words = 0, kept = 0, head_bytes = 0;
+    int threads = 64;
+    for (int v = 0; v < nvol; ++v) {
+        const OnchipVolume &V = vols[v];
+        L.first[v + 1] = L.first[v] + V.plan.blocks();
+        words += align256(sizeof(Word) * nwords_of(V.plan, 1));
+        kept += align256(sizeof(float) * int64_t(V.dims[0]) * V.dims[1] * V.dims[2]);
+        threads = std::max(threads, threads_of(V.plan));
+        head_bytes += V.head_bytes;
+    }
+    const int64_t table_bytes = align256(sizeof(OnchipSolve) * kMany);
+    if (nvol < 1 || nvol > kMany || L.first[nvol] > cus || prm->num_iter < 1 ||
+        prm->num_iter >= INT_MAX / 2 || work_bytes < words + table_bytes + 256 + kept)
+        return MH_OK;
+    std::unique_lock<std::mutex> lock(device_lock(ctx->device), std::try_to_lock);
+    if (!lock.owns_lock()) return MH_OK;
+    L.n = nvol;
+    char *base = static_cast<char *>(work);
+    OnchipSolve *table = reinterpret_cast<OnchipSolve *>(base);
+    int *abort = reinterpret_cast<int *>(base + table_bytes);
+    base += table_bytes + 256;
+    char *keep = base + words;
+    for (int v = 0; v < nvol; ++v) {
+        const OnchipVolume &V = vols[v];
+        const int64_t n = int64_t(V.dims[0]) * V.dims[1] * V.dims[2], nwords = nwords_of(V.plan, 1);
+        Args &A = L.a[v];
+        A = args_of(V.plan, V.F, V.dims, prm);
+        A.inbox = reinterpret_cast<Word *>(base);
+        A.parts = A.inbox + nwords - int64_t(V.plan.blocks()) * 2;
+        base += align256(sizeof(Word) * nwords);
+        A.abort = abort;
+        A.solves = table + v;
+        A.nsolves = A.nslots = 1;
+        Few few{};
+        few.s[0] = V.solve;
+        hipLaunchKernelGGL(onchip_prepare_kernel,
+                           dim3(unsigned(std::min<int64_t>(1024, blocks_for(std::max(n, nwords))))),
+                           dim3(kBlock), 0, s, A.inbox, nwords, table + v, few, 1, n,
+                           reinterpret_cast<float *>(keep), abort);
+        keep += align256(sizeof(float) * n);
+    }
+    MH_CHECK_LAUNCH(ctx, "onchip prepare");
+    const void *kernel = reinterpret_cast<const void *>(&cmf_onchip_kernel<8, kAxial, false, false, kMany>);
+    const int lds = lds_bytes(8, kAxial);
+    void *args[] = {&L};
+    MH_CHECK(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(unsigned(L.first[nvol])),
+                                                    dim3(unsigned(threads)), args, unsigned(lds), s);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return MH_OK;
+    }
+    host->resize(size_t(head_bytes));
+    MH_CHECK(ctx, hipMemcpyAsync(host->data(), heads, size_t(head_bytes), hipMemcpyDeviceToHost, s));
+    MH_CHECK(ctx, hipStreamSynchronize(s));
+    *ran = true;
+    for (int v = 0; v < nvol; ++v) {
+        const OnchipVolume &V = vols[v];
+        const int done = *reinterpret_cast<const int *>(host->data() + (reinterpret_cast<char *>(V.solve.done) -
+                                                                        static_cast<char *>(heads)));
+        *ran = *ran && done == V.plan.blocks();
+    }
+    if (*ran) return MH_OK;
+    // a work-group gave up: every volume as it was
+    keep = base;
+    for (int v = 0; v < nvol; ++v) {
+        const int64_t n = int64_t(vols[v].dims[0]) * vols[v].dims[1] * vols[v].dims[2];
+        hipLaunchKernelGGL(onchip_restore_kernel, dim3(blocks_for(n)), dim3(kBlock), 0, s, vols[v].solve.u,
+                           reinterpret_cast<const float *>(keep), n);
+        MH_CHECK_LAUNCH(ctx, "onchip restore");
+        keep += align256(sizeof(float) * n);
+    }
+    return MH_OK;
+}
 
 int64_t onchip_work_bytes(const OnchipPlan &P, int solves, int cus)
 {
@@ -661,7 +823,9 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     const int slots = slots_of(P, nsolves, cus), lds = lds_bytes(P.v, mode);
     const int64_t nwords = nwords_of(P, slots);
     char *base = static_cast<char *>(work);
-    Args A{};
+    ArgsOf<1> L{};
+    Args &A = L.a[0];
+    A = args_of(P, F, dims, prm);
     A.inbox = reinterpret_cast<Word *>(base);
     A.parts = A.inbox + nwords - int64_t(slots) * P.blocks() * 2;
     base += align256(sizeof(Word) * nwords);
@@ -672,34 +836,6 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     A.solves = table;
     A.nsolves = nsolves;
     A.nslots = slots;
-    A.F = F;
-    A.d0 = dims[0];
-    A.d1 = dims[1];
-    A.d2 = dims[2];
-    A.b1 = P.b1;
-    A.b2 = P.b2;
-    A.nt1 = P.nt1;
-    A.nt2 = P.nt2;
-    A.nz = P.nz;
-    A.num_iter = prm->num_iter;
-    A.update = prm->update;
-    A.rcc = prm->rcc;
-    A.inv_rcc = float(1.0 / double(prm->rcc));
-    A.rs0 = prm->rs[0];
-    A.rs1 = prm->rs[1];
-    A.rs2 = prm->rs[2];
-    A.ss0 = prm->ss[0];
-    A.ss1 = prm->ss[1];
-    A.ss2 = prm->ss[2];
-    A.error_bound = prm->error_bound;
-    A.inv_n_rcc = float(1.0 / (double(n) * double(prm->rcc)));
-    A.sq0 = prm->sqev[0];
-    A.sq1 = prm->sqev[1];
-    A.sq2 = prm->sqev[2];
-    A.rq0 = float(1.0 / double(prm->sqev[0]));
-    A.rq1 = float(1.0 / double(prm->sqev[1]));
-    A.rq2 = float(1.0 / double(prm->sqev[2]));
-    A.A = axi_params(prm);
     Few few{};
     if (nsolves <= kFew)
         std::copy(solves, solves + nsolves, few.s);
@@ -710,7 +846,7 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     hipLaunchKernelGGL(onchip_prepare_kernel, dim3(std::max(pb, blocks_for(nsolves))), dim3(kBlock), 0,
                        s, A.inbox, nwords, table, few, nsolves, n, keep, A.abort);
     MH_CHECK_LAUNCH(ctx, "onchip prepare");
-    void *args[] = {&A};
+    void *args[] = {&L};
     MH_CHECK(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(unsigned(slots * P.blocks())),
                                                     dim3(unsigned(threads_of(P))), args,

@@ -2930,6 +2930,99 @@ MH_EXPORT int mh_cmf_solve_ragged(mh_ctx *ctx, float *u, const float *eigs, cons
     return any_nan ? MH_STOPPED_NAN : MH_OK;
 }
 
+MH_EXPORT int mh_cmf_ragged_onchip(mh_ctx *ctx, float *u, const float *eigs, const float *alpha,
+                                   const float *cs, const float *ct, int nvol, const int64_t *vdims,
+                                   const int64_t *voff, const mh_cmf_params *prm, void *work,
+                                   int64_t work_bytes, mh_cmf_result *res, int *solved, void *stream)
+{
+    MH_REQUIRE(ctx, u && eigs && alpha && cs && ct && vdims && voff && prm && work && res && solved,
+               "null pointer");
+    MH_REQUIRE(ctx, (reinterpret_cast<uintptr_t>(work) & 255) == 0, "workspace must be 256-byte aligned");
+    std::fill(solved, solved + std::max(nvol, 0), 0);
+    // what is not for this launch, or wrong, is left to the other solvers
+    if (ctx->sweep_mode != 0 || nvol < 2 || !mh::axi_params(prm).on || prm->num_iter < 1 ||
+        prm->update < 1 || !(prm->rcc > 0.f) || maxcheck_for(prm) > kCritLogMax / 16)
+        return MH_OK;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) {
+        (void)hipGetLastError();
+        return MH_OK;
+    }
+    std::vector<std::pair<int64_t, int64_t>> iv;
+    struct Item {
+        int v;
+        mh::OnchipPlan plan;
+    };
+    std::vector<Item> items;
+    for (int v = 0; v < nvol; ++v) {
+        const int64_t *d = vdims + 3 * v;
+        if (!mh::dims_ok(d) || voff[v] < 0) return MH_OK;
+        iv.push_back({voff[v], voff[v] + d[0] * d[1] * d[2]});
+        if (d[0] * d[1] * d[2] > (int64_t(1) << 21)) continue;
+        const int dims[3] = {int(d[0]), int(d[1]), int(d[2])};
+        const mh::OnchipPlan P = mh::onchip_plan_many(ctx, dims, prm);
+        if (P.v) items.push_back({v, P});
+    }
+    std::sort(iv.begin(), iv.end());
+    for (size_t k = 1; k < iv.size(); ++k)
+        if (iv[k].first < iv[k - 1].second) return MH_OK;  // overlapping volumes
+    // the largest first, each into the first launch with room for it
+    std::stable_sort(items.begin(), items.end(),
+                     [](const Item &a, const Item &b) { return a.plan.blocks() > b.plan.blocks(); });
+    struct Launch {
+        int blocks = 0;
+        std::vector<Item> items;
+    };
+    std::vector<Launch> launches;
+    for (const Item &it : items) {
+        auto l = std::find_if(launches.begin(), launches.end(), [&](const Launch &k) {
+            return k.blocks + it.plan.blocks() <= cus && k.items.size() < mh::kOnchipMany;
+        });
+        if (l == launches.end()) l = launches.insert(launches.end(), Launch{});
+        l->blocks += it.plan.blocks();
+        l->items.push_back(it);
+    }
+    hipStream_t s = (hipStream_t)stream;
+    const int64_t crits = maxcheck_for(prm);
+    const int64_t head = align256(sizeof(int) * kCtrlWords + sizeof(float) * crits);
+    int any_nan = 0;
+    for (const Launch &l : launches) {
+        const int m = int(l.items.size());
+        if (m < 2 || head * m >= work_bytes) continue;  // alone: its own plan is better
+        char *heads = static_cast<char *>(work);
+        std::vector<mh::OnchipVolume> vols;
+        for (int k = 0; k < m; ++k) {
+            const int v = l.items[size_t(k)].v;
+            const int64_t o = voff[v];
+            int *ctrl = reinterpret_cast<int *>(heads + head * k);
+            vols.push_back({l.items[size_t(k)].plan,
+                            mh::OnchipSolve{u + o, alpha + o, ctrl + kStop, ctrl + kNcrit, ctrl + kDone,
+                                            reinterpret_cast<float *>(ctrl + kCtrlWords), int(crits)},
+                            mh::OnchipFields{eigs + 3 * o, cs + o, ct + o, nullptr},
+                            {int(vdims[3 * v]), int(vdims[3 * v + 1]), int(vdims[3 * v + 2])},
+                            head});
+        }
+        std::vector<char> host;
+        bool ran = false;
+        const int rc = mh::onchip_run_many(ctx, vols.data(), m, prm, heads + head * m,
+                                           work_bytes - head * m, heads, s, &host, &ran);
+        if (rc) return rc;
+        for (int k = 0; ran && k < m; ++k) {
+            const int v = l.items[size_t(k)].v;
+            const int *ctrl = reinterpret_cast<const int *>(host.data() + head * k);
+            const float *log = reinterpret_cast<const float *>(ctrl + kCtrlWords);
+            const int nc = int(std::min<int64_t>(ctrl[kNcrit], crits));
+            res[v].stopped = ctrl[kStop];
+            res[v].ncrit = nc;
+            res[v].iterations = ctrl[kStop] ? (ctrl[kNcrit] - 1) * prm->update + 1 : prm->num_iter;
+            res[v].last_crit = nc > 0 ? log[nc - 1] : 0.f;
+            any_nan |= ctrl[kStop] == 1;
+            solved[v] = 1;
+        }
+    }
+    return any_nan ? MH_STOPPED_NAN : MH_OK;
+}
+
 MH_EXPORT int mh_cmf_batched_set_schedule(mh_ctx *ctx, int group, int visit)
 {
     MH_REQUIRE(ctx, group >= 0 && group <= kSI && visit >= 0, "group in 0..8, visit >= 0");

@@ -213,28 +213,49 @@ class CmfCutQAnisotropicGpu(TreePrintable):
         u = dev.download(t_u)
         return [u[o:o + sz].reshape(s) for o, sz, s in zip(offs, sizes, shapes)]
 
+    def _solve_side_by_side(self, u, quats, alpha, cs, ct, shapes, offsets, sq, scaling):
+        """Per volume its result if it was solved beside others on the chip, else None."""
+        dev, nv = self.loader, len(shapes)
+        if nv < 2:
+            return [None] * nv
+        P = self._cmf_params((1, 1, 1) if scaling is None else scaling, sq, max(1, u.numel()))
+        vd = np.ascontiguousarray(np.asarray(shapes, np.int64).reshape(nv, 3))
+        vo = np.ascontiguousarray(np.asarray(offsets, np.int64))
+        work = dev.bytes(_lib.CMF_RAGGED_ONCHIP_BYTES)
+        res, solved = (_lib.CmfResult * nv)(), np.zeros(nv, np.int32)
+        rc = dev.lib.mh_cmf_ragged_onchip(dev.handle, dev.ptr(u), dev.ptr(quats), dev.ptr(alpha),
+                                          dev.ptr(cs), dev.ptr(ct), nv,
+                                          vd.ctypes.data_as(C.c_void_p),
+                                          vo.ctypes.data_as(C.c_void_p), C.byref(P), dev.ptr(work),
+                                          _lib.CMF_RAGGED_ONCHIP_BYTES, res,
+                                          solved.ctypes.data_as(C.c_void_p), dev.stream)
+        dev.check(rc, "mh_cmf_ragged_onchip")
+        return [res[v] if solved[v] else None for v in range(nv)]
+
     def execute_ragged_device(self, u, quats, alpha, cs, ct, shapes, offsets, eigs, scaling=None,
                               sweep_min_voxels=1 << 19):
-        """Volumes of at least sweep_min_voxels voxels are solved one at a
-        time with the tuned single-solve method (the multi-level sweep where it
-        wins), the others together in one packed launch sequence; both give
-        the same iterations bit for bit (None: all packed)."""
+        """Volumes that fit the chip together share launches there; of the
+        others those of at least sweep_min_voxels voxels are solved one at a
+        time with the tuned single-solve method, the rest together in one packed
+        launch sequence; all give the same iterations bit for bit (None: all
+        packed)."""
         dev = self.loader
         shapes = [tuple(int(v) for v in s) for s in shapes]
         offsets = [int(o) for o in offsets]
         sizes = [int(np.prod(s)) for s in shapes]
-        big = [v for v in range(len(shapes))
-               if sweep_min_voxels is not None and sizes[v] >= sweep_min_voxels]
-        if big:
+        if sweep_min_voxels is not None and shapes:
             sq = np.sqrt(np.asarray(eigs, dtype=np.float64))
-            results = [None] * len(shapes)
-            for v in big:
+            results = self._solve_side_by_side(u, quats, alpha, cs, ct, shapes, offsets, sq, scaling)
+            rest = [v for v in range(len(shapes)) if results[v] is None]
+            for v in rest:
+                if sizes[v] < sweep_min_voxels:
+                    continue
                 o, m = offsets[v], sizes[v]
                 self.execute_device(u[o:o + m], quats[3 * o:3 * (o + m)], alpha[o:o + m],
                                     cs[o:o + m], ct[o:o + m], scaling=scaling, const_sqevals=sq,
                                     shape=shapes[v])
                 results[v] = self.last_result
-            small = [v for v in range(len(shapes)) if v not in set(big)]
+            small = [v for v in rest if sizes[v] < sweep_min_voxels]
             if small:
                 self.execute_ragged_device(u, quats, alpha, cs, ct, [shapes[v] for v in small],
                                            [offsets[v] for v in small], eigs, scaling, None)
