@@ -1,6 +1,8 @@
 // Gradient vector flow on gfx950: explicit-Euler steps on the three SoA
 // components, ping-ponging two buffers, mirrored neighbours at the faces;
 // one step per launch, or two to four per launch in a sweep along axis 0.
+#include <algorithm>
+
 #include "cmf_words.h"
 #include "mh_common.h"
 #include "mh_reduce.h"
@@ -328,13 +330,17 @@ GvfPlan gvf_plan(mh_ctx *ctx, const int64_t dims[3], int iters, int64_t max_grou
         cus <= 0)
         cus = 256;
     double cost = any ? 1e30 : 2.2 + 5.6e-6 * double(dims[0]) * double(dims[1]) * double(dims[2]);
+    if (cost < 3.0) return best;  // no sweep takes less
     const int d0 = int(dims[0]);
     for (const GvfShape &S : kGvfShapes) {
         if (iters < S.levels) continue;
         const int64_t tiles = ((dims[2] + S.tx - 1) / S.tx) * ((dims[1] + S.ty - 1) / S.ty);
-        for (int z = 1; z <= d0; ++z) {
+        // as many chunks as fill the device once, twice, ..
+        for (int64_t waves = (tiles + cus - 1) / cus, k = 0; k < 8; ++waves, ++k) {
+            const int chunks = int(std::min<int64_t>(d0, waves * cus / tiles));
+            const int z = (d0 + chunks - 1) / chunks;
             const int64_t groups = tiles * ((d0 + z - 1) / z);
-            if (groups > max_groups) continue;
+            if (groups > max_groups) break;
             const double c = (double((groups + cus - 1) / cus) * (z + 2 * (S.levels - 1)) * S.unit + 2.5) /
                              S.levels;
             if (c < cost) {
