@@ -534,13 +534,16 @@ SlidePlan slide_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, b
             }
         }
     }
-    // Where it wins: against the sweeps, which do 0.95e11 .. 1.35e11 voxels and
-    // iterations a second (256^3 1.22e11 against 2.18e11 here, 192^3 1.28e11 and
-    // 1.49e11, 320^3 0.94e11 and 1.36e11; but 150 x 128 x 141 1.34e11 and 1.27e11,
-    // 420^3 1.30e11 and 0.92e11, 256^3 with a criterion every 5 iterations 0.97e11
-    // and 0.82e11), and with seeds against the per-iteration kernels (256^3 5.6e10
-    // and 2.08e11, 128 x 512 x 512 5.7e10 and 1.2e11).
-    if (best.levels && best_cost > double(n) / (sup ? 6e4 : 1.35e5)) best.levels = 0;
+    // Where it wins: against the sweeps, which do up to 1.5e11 voxels and iterations
+    // a second while their state stays in the last-level cache (132 x 159 x 155
+    // 1.48e11 against 1.46e11 here) and 0.95e11 .. 1.3e11 beyond it (256^3 1.22e11
+    // against 2.18e11 here, 192^3 1.28e11 and 1.49e11, 240 x 230 x 190 1.17e11 and
+    // 1.63e11, 320^3 1.2e11 and 1.36e11; but 420^3 1.30e11 and 0.92e11, 256^3 with a
+    // criterion every 5 iterations 1.1e11 and 0.82e11), and with seeds against the
+    // per-iteration kernels (256^3 5.6e10 and 2.08e11, 128 x 512 x 512 5.7e10 and
+    // 1.2e11).
+    const double others = sup ? 6e4 : n < (int64_t(1) << 22) ? 1.5e5 : 1.3e5;
+    if (best.levels && best_cost > double(n) / others) best.levels = 0;
     return best;
 }
 
