@@ -25,6 +25,14 @@
 // is bounded: after kWaitSpins loads without its word a work-group raises the abort
 // flag, every wait ends, and the host restores u and solves another way.
 //
+// Bound at 128^3 (one wave of 8 planes per SIMD slot) by the issue of 74 vector
+// instructions per voxel, 3.95 of 4.4 to 4.6 us an iteration (16.0 in the
+// three-level sweep); below about 80^3 by the two exchanges (64^3 2.6 us, 6.1 in
+// the per-iteration kernels). Rows are sent first in their phase and words polled
+// at its end: sent last they cost 0.5 us more, polled by the waves that read them
+// only, after the barrier, 0.5; two work-groups of half the size per compute unit
+// are no faster (96^3 4.1 against 3.7 us).
+//
 // The per-voxel arithmetic is cmf_voxel.h's, so the result equals the
 // per-iteration kernels' bit for bit; the criterion's sum is taken in another
 // order.
@@ -42,12 +50,11 @@ namespace {
 
 using namespace mh;
 
-constexpr int kRedFloats = 64;       // three sets of the waves' sums, the failure flag last
-constexpr int kWords = 2;      // in-plane words a thread receives per phase
-
 constexpr int kMaxThreads = 1024;
-constexpr int kMaxPlanes = 8;  // per thread, constant eigenvalues (l0, l1, l1); else half
-constexpr int kCells = 1184;   // LDS cells of a tile and its faces
+constexpr int kMaxPlanes = 8;   // per thread, constant eigenvalues (l0, l1, l1); else half
+constexpr int kCells = 1184;    // LDS cells of a tile and its faces
+constexpr int kWords = 2;       // in-plane words a thread receives per phase
+constexpr int kRedFloats = 64;  // three sets of the waves' sums, the failure flag last
 
 struct SumOp {
     __device__ static float identity() { return 0.f; }
