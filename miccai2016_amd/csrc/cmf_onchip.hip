@@ -25,12 +25,12 @@
 // is bounded: after kWaitSpins loads without its word a work-group raises the abort
 // flag, every wait ends, and the host restores u and solves another way.
 //
-// Bound at 128^3 by the issue of 74 vector instructions per voxel, 3.95 of 4.4 to 4.6 us an iteration (16.0 in the
-// three-level sweep); below about 80^3 by the two exchanges (64^3 2.6 us, 6.1 in
-// the per-iteration kernels). Words are polled as their phase ends, by all threads:
-// polled after the barrier by the waves that read them 5.3 us at 128^3 (4.8 in the
-// same run); two work-groups of half the size per compute unit
-// are no faster (96^3 4.1 against 3.7 us).
+// Bound at 128^3 by the issue of 74 vector instructions per voxel, 3.95 of 4.4 to
+// 4.6 us an iteration (16.0 in the three-level sweep); below about 80^3 by the two
+// exchanges (64^3 2.6 us, 6.1 in the per-iteration kernels). Words are polled as
+// their phase ends, by all threads: polled after the barrier by the waves that
+// read them 5.3 us at 128^3 (4.8 in the same run); two work-groups of half the size
+// per compute unit are no faster (96^3 4.1 against 3.7 us).
 //
 // The per-voxel arithmetic is cmf_voxel.h's, so the result equals the
 // per-iteration kernels' bit for bit; the criterion's sum is taken in another
