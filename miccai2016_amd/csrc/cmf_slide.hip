@@ -312,7 +312,10 @@ cmf_slide_kernel(const Args A)
             over0 = (unsigned(__ballot(k > 0)) & 1u) != 0;
         }
         const unsigned act = adv & kMine, out = mask >> 8 & kMine;
-        const int joins = s < A.d0 ? ph - 1 : -1, settles = s <= A.d0 && s > 0 ? ph - 2 : -1;
+        // planes s, s - 1 and s - 2 levels: their positions, from 0 to W - 1 (of this
+        // run's if below kRun; with one run per tile, W = kRun, all of them are)
+        const int joins = s < A.d0 ? (ph >= 1 ? ph - 1 : W - 1) : -1;
+        const int settles = s <= A.d0 && s > 0 ? (ph >= 2 ? ph - 2 : ph - 2 + W) : -1;
         const int leaves = s >= lv2 ? (ph - 1 < lv2 ? ph - 1 - lv2 + W : ph - 1 - lv2) : -1;
         lds_barrier();
         Vec4 *own = own_cell(t8);
