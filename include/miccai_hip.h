@@ -379,7 +379,7 @@ int mh_cmf_batched_set_sweep(mh_ctx *ctx, int mode);
  * of that otherwise) stays on the chip from its first iteration to its last,
  * unless another such solve is running on the device. On the same condition a
  * larger one with eigenvalues (l0, l1, l1) goes through the volume with a
- * sliding window of planes, up to 31 iterations a pass, where that is faster
+ * sliding window of planes, several iterations a pass, where that is faster
  * (measured: 256^3 1.8 times, with seeds 3.8 times). What follows is for the
  * others. Unsupervised constant-eigenvalue solves may advance two, three
  * or four iterations per pass over the state (temporal blocking along axis
@@ -394,6 +394,13 @@ int mh_cmf_batched_set_sweep(mh_ctx *ctx, int mode);
  * chunk a cost model of the launch favours for that tile shape).
  * Results do not depend on any of them, bit for bit. */
 int mh_cmf_set_sweep(mh_ctx *ctx, int mode, int tile, int zchunk);
+/* How such passes cut a volume on a device of so many compute units (no counterpart
+ * in the reference; host arithmetic only, no context): returns the iterations of a
+ * pass, 0 where other methods are taken, and sets plan (may be NULL) to the voxels
+ * of a tile along axes 1 and 2, the tiles along them, the runs of 8 planes a
+ * window has and the bytes of LDS a work-group takes. */
+int mh_cmf_slide_plan(const int64_t dims[3], const mh_cmf_params *params, int seeded,
+                      int compute_units, int plan[6]);
 /* Graph replay in mh_cmf_solve and the resident solves (no counterpart in the
  * reference): when the per-iteration kernels run, one criterion cycle (update
  * iterations starting at a criterion iteration) is captured as a HIP graph

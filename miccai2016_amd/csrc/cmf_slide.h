@@ -16,8 +16,11 @@ struct SlidePlan {
 };
 
 // The plan for solves of these dims (with seeds: `sup`) whose criterion comes
-// every `update` iterations.
+// every `update` iterations, on this context's device or one of so many compute
+// units; the bytes of LDS a work-group of it takes.
 SlidePlan slide_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, bool sup);
+SlidePlan slide_plan(int compute_units, const int dims[3], const mh_cmf_params *prm, bool sup);
+int slide_lds_bytes(const SlidePlan &plan);
 
 // Device bytes of the words its work-groups exchange.
 int64_t slide_inbox_bytes(const SlidePlan &plan);

@@ -35,6 +35,7 @@
 //
 // The per-voxel arithmetic is cmf_voxel.h's, so the result equals the
 // per-iteration kernels' bit for bit.
+#include <algorithm>
 #include <mutex>
 
 #include "cmf_slide.h"
@@ -70,6 +71,9 @@ struct Addresses {  // SlideFields, as kept in LDS
 };
 constexpr int kLdsFixed = 16 * kLdsVecs + 4 * kRedFloats + 4 * kMaxThreads + int(sizeof(Addresses));
 int lds_bytes(int slots) { return kLdsFixed + 4 * kRun * slots; }
+// what the masks may take of a compute unit's LDS (block_reduce holds 64 bytes)
+constexpr int kLds = 160 * 1024, kLdsReduce = 64;
+constexpr int kMaxSlots = (kLds - kLdsReduce - kLdsFixed) / (4 * kRun);
 
 struct Args {
     SlideFields F;
@@ -497,13 +501,12 @@ int64_t slide_inbox_bytes(const SlidePlan &P)
     return int64_t(P.blocks()) * 16 * (int64_t(P.b1) * P.b2 + 8 * (P.b1 + P.b2));
 }
 
-SlidePlan slide_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, bool sup)
+SlidePlan slide_plan(int cus, const int dims[3], const mh_cmf_params *prm, bool sup)
 {
     SlidePlan best;
     const int64_t n = int64_t(dims[0]) * dims[1] * dims[2];
     // byte offsets of the AoS x4 frames stay below 2^31
-    if (!axi_params(prm).on || n >= (int64_t(1) << 27) || ctx->device >= kMaxDevices) return best;
-    const int cus = compute_units(ctx);
+    if (!axi_params(prm).on || n >= (int64_t(1) << 27)) return best;
     double best_cost = 0;
     for (int n2 = 1; n2 <= std::min(dims[2], 16); ++n2) {
         const int b2 = (dims[2] + n2 - 1) / n2;
@@ -519,7 +522,7 @@ SlidePlan slide_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, b
             if (tiles > cus || P.b1 * b2 + P.b1 + b2 + 1 > kCells)
                 continue;
             // W = 8 slots planes hold 4 slots - 1 levels; a pass ends at a criterion
-            P.slots = std::min(cus / tiles, (prm->update + 4) / 4);
+            P.slots = std::min({cus / tiles, (prm->update + 4) / 4, kMaxSlots});
             P.levels = std::min(4 * P.slots - 1, prm->update);
             const int passes = (prm->update + P.levels - 1) / P.levels;
             P.levels = (prm->update + passes - 1) / passes;
@@ -549,6 +552,13 @@ SlidePlan slide_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, b
     if (best.levels && best_cost > double(n) / others) best.levels = 0;
     return best;
 }
+
+SlidePlan slide_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, bool sup)
+{
+    return ctx->device < kMaxDevices ? slide_plan(compute_units(ctx), dims, prm, sup) : SlidePlan();
+}
+
+int slide_lds_bytes(const SlidePlan &P) { return lds_bytes(P.slots) + kLdsReduce; }
 
 int slide_pass(mh_ctx *ctx, const SlidePlan &P, const SlideFields &F, const int dims[3],
                const mh_cmf_params *prm, int lv, int it, bool check, int cur, const SlideControl &C,
@@ -602,3 +612,16 @@ int slide_pass(mh_ctx *ctx, const SlidePlan &P, const SlideFields &F, const int 
 }
 
 }  // namespace mh
+
+MH_EXPORT int mh_cmf_slide_plan(const int64_t dims[3], const mh_cmf_params *prm, int seeded,
+                                int compute_units, int plan[6])
+{
+    if (!mh::dims_ok(dims) || !prm || prm->update < 1) return MH_ERR_ARG;
+    const int d[3] = {int(dims[0]), int(dims[1]), int(dims[2])};
+    const mh::SlidePlan P = mh::slide_plan(compute_units, d, prm, seeded != 0);
+    if (P.levels && plan) {
+        const int v[6] = {P.b1, P.b2, P.nt1, P.nt2, P.slots, mh::slide_lds_bytes(P)};
+        std::copy(v, v + 6, plan);
+    }
+    return P.levels;
+}

@@ -16,3 +16,14 @@ def test_one_run_of_planes_per_tile(dev, shape, iters):
     want = _solve(dev, f, shape, 1, iters, 30)
     assert dev.torch.equal(got[0], want[0])
     assert got[1] == want[1]
+
+
+def test_long_windows(dev):
+    """One tile and a rare criterion: hundreds of iterations a pass."""
+    shape = (4000, 32, 32)
+    f = _fields(dev, shape, "axial")
+    print(shape, flush=True)
+    got = _solve(dev, f, shape, 0, 1010, 1000)
+    want = _solve(dev, f, shape, 1, 1010, 1000)
+    assert dev.torch.equal(got[0], want[0])
+    assert got[1] == want[1]
