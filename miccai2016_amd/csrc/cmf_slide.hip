@@ -507,6 +507,9 @@ SlidePlan slide_plan(int cus, const int dims[3], const mh_cmf_params *prm, bool 
     const int64_t n = int64_t(dims[0]) * dims[1] * dims[2];
     // byte offsets of the AoS x4 frames stay below 2^31
     if (!axi_params(prm).on || n >= (int64_t(1) << 27)) return best;
+    // (a window of cus runs of planes holds 4 cus - 1 iterations: a criterion rarer
+    // than that, INT_MAX among them, ends no pass)
+    const int update = std::min(prm->update, 4 * std::max(cus, 1));
     double best_cost = 0;
     for (int n2 = 1; n2 <= std::min(dims[2], 16); ++n2) {
         const int b2 = (dims[2] + n2 - 1) / n2;
@@ -522,10 +525,10 @@ SlidePlan slide_plan(int cus, const int dims[3], const mh_cmf_params *prm, bool 
             if (tiles > cus || P.b1 * b2 + P.b1 + b2 + 1 > kCells)
                 continue;
             // W = 8 slots planes hold 4 slots - 1 levels; a pass ends at a criterion
-            P.slots = std::min({cus / tiles, (prm->update + 4) / 4, kMaxSlots});
-            P.levels = std::min(4 * P.slots - 1, prm->update);
-            const int passes = (prm->update + P.levels - 1) / P.levels;
-            P.levels = (prm->update + passes - 1) / passes;
+            P.slots = std::min({cus / tiles, (update + 4) / 4, kMaxSlots});
+            P.levels = std::min(4 * P.slots - 1, update);
+            const int passes = (update + P.levels - 1) / P.levels;
+            P.levels = (update + passes - 1) / passes;
             P.slots = std::min(P.slots, (P.levels + 4) / 4);
             if (P.levels < 3) continue;
             const int waves = (threads_of(P) / 64 + 3) / 4;

@@ -27,3 +27,14 @@ def test_long_windows(dev):
     want = _solve(dev, f, shape, 1, 1010, 1000)
     assert dev.torch.equal(got[0], want[0])
     assert got[1] == want[1]
+
+
+def test_no_criterion_after_the_first(dev):
+    """The largest interval between criteria."""
+    shape = (132, 160, 160)
+    f = _fields(dev, shape, "seeded")
+    print(shape, flush=True)
+    got = _solve(dev, f, shape, 0, 20, 2 ** 31 - 1)
+    want = _solve(dev, f, shape, 1, 20, 2 ** 31 - 1)
+    assert dev.torch.equal(got[0], want[0])
+    assert got[1] == want[1] and len(got[2]) == 1
