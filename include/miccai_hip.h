@@ -401,6 +401,14 @@ int mh_cmf_set_sweep(mh_ctx *ctx, int mode, int tile, int zchunk);
  * window has and the bytes of LDS a work-group takes. */
 int mh_cmf_slide_plan(const int64_t dims[3], const mh_cmf_params *params, int seeded,
                       int compute_units, int plan[6]);
+/* The compute units that solves on the chip and sliding passes are planned for (no
+ * counterpart in the reference): 0 (default) the device's, fewer leave the others to
+ * work on other streams. More than the device has make launches that it refuses;
+ * such solves take other methods. Results do not depend on it, bit for bit. */
+int mh_cmf_set_chip_units(mh_ctx *ctx, int units);
+/* On this context so far: solves finished on the chip, sliding passes launched, and
+ * launches of either that the device refused. */
+int mh_cmf_chip_counts(mh_ctx *ctx, int64_t counts[3]);
 /* Graph replay in mh_cmf_solve and the resident solves (no counterpart in the
  * reference): when the per-iteration kernels run, one criterion cycle (update
  * iterations starting at a criterion iteration) is captured as a HIP graph

@@ -537,16 +537,6 @@ int words_of(const mh::OnchipPlan &P)  // in-plane face words of a brick
 
 int threads_of(const mh::OnchipPlan &P) { return (P.b1 * P.b2 + 63) / 64 * 64; }
 
-int compute_units(mh_ctx *ctx)
-{
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) {
-        (void)hipGetLastError();
-        cus = 0;
-    }
-    return cus;
-}
-
 template <int V, int MODE, bool DEFER>
 const void *kernel_sup(bool sup)
 {
@@ -606,6 +596,17 @@ std::mutex g_device_mu[kMaxDevices];
 namespace mh {
 
 std::mutex &device_lock(int device) { return g_device_mu[device]; }
+
+int compute_units(mh_ctx *ctx)
+{
+    int cus = 0;
+    if (ctx->chip_units > 0) return ctx->chip_units;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) {
+        (void)hipGetLastError();
+        cus = 0;
+    }
+    return cus;
+}
 
 OnchipPlan onchip_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, int solves)
 {
@@ -776,6 +777,7 @@ int onchip_run_many(mh_ctx *ctx, const OnchipVolume *vols, int nvol, const mh_cm
                                                     dim3(unsigned(threads)), args, unsigned(lds), s);
     if (e != hipSuccess) {
         (void)hipGetLastError();
+        ++ctx->chip.refused;
         return MH_OK;
     }
     host->resize(size_t(head_bytes));
@@ -788,7 +790,10 @@ int onchip_run_many(mh_ctx *ctx, const OnchipVolume *vols, int nvol, const mh_cm
                                                                         static_cast<char *>(heads)));
         *ran = *ran && done == V.plan.blocks();
     }
-    if (*ran) return MH_OK;
+    if (*ran) {
+        ctx->chip.solves += nvol;
+        return MH_OK;
+    }
     // a work-group gave up: every volume as it was
     keep = base;
     for (int v = 0; v < nvol; ++v) {
@@ -859,6 +864,7 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
                                                     unsigned(lds), s);
     if (e != hipSuccess) {  // the device does not hold every work-group: nothing ran
         (void)hipGetLastError();
+        ++ctx->chip.refused;
         return MH_OK;
     }
     // every solve's done word counts the bricks that stored u
@@ -874,6 +880,7 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     *ran = true;
     for (int q = 0; q < nsolves; ++q) {
         done[size_t(q)] = done[size_t(q)] == P.blocks();
+        ctx->chip.solves += done[size_t(q)];
         if (done[size_t(q)]) continue;
         *ran = false;
         hipLaunchKernelGGL(onchip_restore_kernel, dim3(blocks_for(n)), dim3(kBlock), 0, s, solves[q].u,

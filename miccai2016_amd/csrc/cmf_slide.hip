@@ -480,16 +480,6 @@ __global__ void __launch_bounds__(mh::kBlock) zero_words_kernel(Word *w, int64_t
     if (i < n) w[i] = 0;
 }
 
-int compute_units(mh_ctx *ctx)
-{
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) {
-        (void)hipGetLastError();
-        cus = 0;
-    }
-    return cus;
-}
-
 int threads_of(const SlidePlan &P) { return (P.b1 * P.b2 + 63) / 64 * 64; }
 
 }  // namespace

@@ -20,6 +20,10 @@ constexpr int kWaitSpins = 1 << 16;  // loads of a word that does not come: tens
 constexpr int kMaxDevices = 64;
 std::mutex &device_lock(int device);  // cmf_onchip.hip
 
+// Compute units that plans for such launches count on: the device's, or what
+// mh_cmf_set_chip_units says; 0 if they are not known.
+int compute_units(mh_ctx *ctx);
+
 template <int G>
 struct alignas(4 * G) Vec {
     float v[G];

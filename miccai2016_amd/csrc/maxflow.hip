@@ -1474,7 +1474,12 @@ struct Runner {
             }
             const bool chk = ((it + lv - 1) % prm->update) == 0;
             slide_rc = slide_step(lv, chk);
-            if (slide_rc) return 0;  // nothing was launched
+            if (slide_rc) {  // nothing was launched; the error is not this solve's
+                (void)hipGetLastError();
+                ++ctx->chip.refused;
+                return 0;
+            }
+            ++ctx->chip.passes;
             if (chk)
                 hipLaunchKernelGGL(cmf_crit_kernel, dim3(1), dim3(1024), 0, s, W.partials, slide.blocks(),
                                    UP.inv_n_rcc, UP.error_bound, W.ctrl, W.crit_log);
@@ -2943,11 +2948,7 @@ MH_EXPORT int mh_cmf_ragged_onchip(mh_ctx *ctx, float *u, const float *eigs, con
     if (ctx->sweep_mode != 0 || nvol < 2 || !mh::axi_params(prm).on || prm->num_iter < 1 ||
         prm->update < 1 || !(prm->rcc > 0.f) || maxcheck_for(prm) > kCritLogMax / 16)
         return MH_OK;
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess) {
-        (void)hipGetLastError();
-        return MH_OK;
-    }
+    const int cus = mh::compute_units(ctx);
     std::vector<std::pair<int64_t, int64_t>> iv;
     struct Item {
         int v;
@@ -3066,6 +3067,25 @@ MH_EXPORT int mh_cmf_batched_sweep_choice(mh_ctx *ctx, const int64_t dims[3], in
     *tile = f->second.first + 1;
     *zchunk = f->second.second;
     return 1;
+}
+
+MH_EXPORT int mh_cmf_set_chip_units(mh_ctx *ctx, int units)
+{
+    if (!ctx) return MH_ERR_ARG;
+    MH_REQUIRE(ctx, units >= 0, "units >= 0");
+    ctx->chip_units = units;
+    ctx->onchip_plans.clear();
+    return MH_OK;
+}
+
+MH_EXPORT int mh_cmf_chip_counts(mh_ctx *ctx, int64_t counts[3])
+{
+    if (!ctx) return MH_ERR_ARG;
+    MH_REQUIRE(ctx, counts, "null pointer");
+    counts[0] = ctx->chip.solves;
+    counts[1] = ctx->chip.passes;
+    counts[2] = ctx->chip.refused;
+    return MH_OK;
 }
 
 MH_EXPORT int mh_cmf_set_graphs(mh_ctx *ctx, int on)

@@ -56,6 +56,12 @@ struct mh_ctx {
     // method the batched solver's tuner chose per volume dims (tile shape,
     // plane chunk), timed on pairs of solves
     std::map<std::array<int, 3>, std::pair<int, int>> batch_tuned;
+    // compute units that plans of solves on the chip and of sliding passes count
+    // on (0: the device's), and what became of them (mh_cmf_chip_counts)
+    int chip_units = 0;
+    struct {
+        int64_t solves = 0, passes = 0, refused = 0;
+    } chip;
     // bricks of the on-chip solver per (dims, p-step form, solves)
     std::map<std::array<int, 5>, std::array<int, 6>> onchip_plans;
     // words the work-groups of the sliding passes exchange (grown on demand),
