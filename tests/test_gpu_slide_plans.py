@@ -2,7 +2,9 @@
 kernels bit for bit."""
 import pytest
 
+from test_gpu_chip_fallbacks import _counts
 from test_gpu_onchip import _fields, _solve
+from test_slide_plan import _plan
 
 pytestmark = pytest.mark.gpu
 
@@ -38,3 +40,30 @@ def test_no_criterion_after_the_first(dev):
     want = _solve(dev, f, shape, 1, 20, 2 ** 31 - 1)
     assert dev.torch.equal(got[0], want[0])
     assert got[1] == want[1] and len(got[2]) == 1
+
+
+@pytest.mark.parametrize("shape,kind,iters,update,levels,slots", [
+    ((10, 500, 500), "seeded", 33, 30, 3, 1),      # one run of planes, two columns of tiles
+    ((80, 500, 501), "seeded", 25, 30, 3, 1),      # columns one voxel short
+    ((17, 300, 290), "seeded", 40, 30, 6, 2),
+    ((33, 256, 256), "seeded", 40, 30, 15, 4),     # little more than one window
+    ((33, 256, 256), "seeded", 7, 30, 15, 4),      # one short pass
+    ((300, 33, 1025), "seeded", 40, 30, 15, 4),    # three columns of tiles
+    ((130, 160, 160), "axial", 62, 30, 30, 8),     # eight runs of planes
+    ((700, 64, 65), "seeded", 125, 60, 60, 16),
+])
+def test_plans_equal_per_iteration_kernels(dev, shape, kind, iters, update, levels, slots):
+    cus = dev.torch.cuda.get_device_properties(dev.device).multi_processor_count
+    plan = _plan(shape, update, kind == "seeded", cus)
+    if cus == 256:
+        assert (plan[0], plan[3]) == (levels, slots)
+    f = _fields(dev, shape, kind)
+    print(shape, kind, plan, flush=True)
+    at = _counts(dev)
+    got = _solve(dev, f, shape, 0, iters, update)
+    solves, passes, refused = _counts(dev) - at
+    # of three iterations or more each
+    assert solves == refused == 0 and 1 <= passes <= iters // 3 and passes >= (iters - 2) // levels
+    want = _solve(dev, f, shape, 1, iters, update)
+    assert dev.torch.equal(got[0], want[0])
+    assert got[1] == want[1]
