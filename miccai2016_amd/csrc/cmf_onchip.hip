@@ -468,8 +468,11 @@ cmf_onchip_kernel(const ArgsOf<N> L)
         }
         if (DEFER && pending) crit_settle();
         ++tag;
+        // read before the barrier (every wait of this solve is behind an earlier one):
+        // after it, a wave ahead may give up in the next solve
+        const int failed = *fail;
         lds_barrier();
-        if (*fail) return;
+        if (failed) return;
         const mh::OnchipSolve &S = A.solves[here_s(q)];
         if (inv) {
             float *out = S.u;
