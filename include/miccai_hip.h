@@ -406,9 +406,16 @@ int mh_cmf_slide_plan(const int64_t dims[3], const mh_cmf_params *params, int se
  * work on other streams. More than the device has make launches that it refuses;
  * such solves take other methods. Results do not depend on it, bit for bit. */
 int mh_cmf_set_chip_units(mh_ctx *ctx, int units);
-/* On this context so far: solves finished on the chip, sliding passes launched, and
- * launches of either that the device refused. */
-int mh_cmf_chip_counts(mh_ctx *ctx, int64_t counts[3]);
+/* On this context so far: solves finished on the chip, sliding passes launched,
+ * launches of either that the device refused, and launches on the chip and solves in
+ * sliding passes that were given up: a work-group waits some tens of milliseconds for
+ * what another sends (another process on the same device may keep that from running);
+ * then the launch ends, its solves are as before it and take other methods. */
+int mh_cmf_chip_counts(mh_ctx *ctx, int64_t counts[4]);
+/* For tests of that: from solve `from` of a launch on the chip, and from sliding pass
+ * `from` of a solve, one work-group is missing (-1, the default: none is). Results do
+ * not depend on it, bit for bit. */
+int mh_cmf_set_lost_group(mh_ctx *ctx, int from);
 /* Graph replay in mh_cmf_solve and the resident solves (no counterpart in the
  * reference): when the per-iteration kernels run, one criterion cycle (update
  * iterations starting at a criterion iteration) is captured as a HIP graph

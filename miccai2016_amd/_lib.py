@@ -124,7 +124,8 @@ SIGNATURES = {
     "mh_cmf_solve_ragged": (i32, [vp, vp, vp, vp, vp, vp, i32, vp, vp, C.POINTER(CmfParams), vp,
                                   i64, C.POINTER(CmfResult), vp]),
     "mh_cmf_set_chip_units": (i32, [vp, i32]),
-    "mh_cmf_chip_counts": (i32, [vp, C.POINTER(i64 * 3)]),
+    "mh_cmf_set_lost_group": (i32, [vp, i32]),
+    "mh_cmf_chip_counts": (i32, [vp, C.POINTER(i64 * 4)]),
     "mh_cmf_slide_plan": (i32, [I64x3, C.POINTER(CmfParams), i32, i32, vp]),
     "mh_cmf_ragged_onchip": (i32, [vp, vp, vp, vp, vp, vp, i32, vp, vp, C.POINTER(CmfParams), vp,
                                    i64, C.POINTER(CmfResult), vp, vp]),

@@ -68,6 +68,7 @@ constexpr int kPointwise = 2;  // eigenvalues of their own at every voxel
 struct Args {
     const mh::OnchipSolve *solves;
     int nsolves, nslots;
+    int nfirst;  // solves the first brick takes part in: all (mh_cmf_set_lost_group: fewer)
     mh::OnchipFields F;
     int d0, d1, d2;
     int b1, b2, nt1, nt2, nz;
@@ -243,7 +244,8 @@ cmf_onchip_kernel(const ArgsOf<N> L)
 
     unsigned tag = 1;
     int nparts = 0;
-    for (int q = slot; q < A.nsolves; q += A.nslots) {
+    const int nsolves = lb == 0 ? A.nfirst : A.nsolves;
+    for (int q = slot; q < nsolves; q += A.nslots) {
         float h0[V], h1[V], h2[V], pt[V], u[V], al[V], cs[V], ct[V], fr[V][NF];
         unsigned lab = 0;
         {
@@ -660,6 +662,10 @@ int64_t nwords_of(const OnchipPlan &P, int slots)
 {
     return int64_t(slots) * P.blocks() * (2 * (P.b1 * P.b2 + words_of(P)) + 2);
 }
+int first_brick_solves(mh_ctx *ctx, int solves)
+{
+    return ctx->lost_group < 0 ? solves : std::min(ctx->lost_group, solves);
+}
 Args args_of(const OnchipPlan &P, const OnchipFields &F, const int dims[3], const mh_cmf_params *prm)
 {
     Args A{};
@@ -763,6 +769,7 @@ int onchip_run_many(mh_ctx *ctx, const OnchipVolume *vols, int nvol, const mh_cm
         A.abort = abort;
         A.solves = table + v;
         A.nsolves = A.nslots = 1;
+        A.nfirst = first_brick_solves(ctx, 1);
         Few few{};
         few.s[0] = V.solve;
         hipLaunchKernelGGL(onchip_prepare_kernel,
@@ -798,6 +805,7 @@ int onchip_run_many(mh_ctx *ctx, const OnchipVolume *vols, int nvol, const mh_cm
         return MH_OK;
     }
     // a work-group gave up: every volume as it was
+    ++ctx->chip.given_up;
     keep = base;
     for (int v = 0; v < nvol; ++v) {
         const int64_t n = int64_t(vols[v].dims[0]) * vols[v].dims[1] * vols[v].dims[2];
@@ -850,6 +858,7 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     A.solves = table;
     A.nsolves = nsolves;
     A.nslots = slots;
+    A.nfirst = first_brick_solves(ctx, nsolves);
     Few few{};
     if (nsolves <= kFew)
         std::copy(solves, solves + nsolves, few.s);
@@ -890,6 +899,7 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
                            keep + q * n, n);
         MH_CHECK_LAUNCH(ctx, "onchip restore");
     }
+    ctx->chip.given_up += !*ran;
     if (finished) finished->swap(done);
     return MH_OK;
 }

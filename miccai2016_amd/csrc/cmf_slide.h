@@ -46,9 +46,10 @@ constexpr int kSlideAborted = 3;
 // Enqueue one pass of lv (1 .. plan.levels) iterations from iteration `it`; the
 // device lock must be held until it is done. With `check`, partials[block]
 // receives each work-group's sum of |err| of the last iteration. The tags of
-// the pass follow *tags, which it advances (0: the inbox is new).
+// the pass follow *tags, which it advances (0: the inbox is new). `lost`: one of
+// its work-groups is missing.
 int slide_pass(mh_ctx *ctx, const SlidePlan &plan, const SlideFields &F, const int dims[3],
-               const mh_cmf_params *prm, int lv, int it, bool check, int cur, const SlideControl &C,
-               float *partials, void *inbox, unsigned *tags, hipStream_t s);
+               const mh_cmf_params *prm, int lv, int it, bool check, int cur, bool lost,
+               const SlideControl &C, float *partials, void *inbox, unsigned *tags, hipStream_t s);
 
 }  // namespace mh

@@ -80,7 +80,7 @@ struct Args {
     SlideControl C;
     int d0, d1, d2;
     int b1, b2, nt1, nt2, slots;
-    int levels, it, check, cur;
+    int levels, it, check, cur;  // check & 2: the last work-group is missing
     float rcc, inv_rcc, rs0, rs1, rs2, ss0, ss1, ss2;
     AxiParams A;
     Word *inbox;  // per work-group: [axis-0 residuals | h0 | rows and columns of residuals | of h]
@@ -112,7 +112,7 @@ template <bool SUP>
 __global__ void __launch_bounds__(kMaxThreads)
 cmf_slide_kernel(const Args A)
 {
-    if (*A.C.stop) return;
+    if (*A.C.stop || ((A.check & 2) && blockIdx.x > 0 && blockIdx.x == gridDim.x - 1)) return;
     using Vec4 = Vec<4>;
     using Vec2 = Vec<2>;
     extern __shared__ __align__(16) unsigned char lds[];
@@ -470,7 +470,7 @@ cmf_slide_kernel(const Args A)
         *A.C.stop = kSlideAborted;
         return;
     }
-    if (A.check) A.partials[b] = aerr;
+    if (A.check & 1) A.partials[b] = aerr;
     if (b == 0) *A.C.parity = 1 - A.cur;
 }
 
@@ -554,8 +554,8 @@ SlidePlan slide_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm, b
 int slide_lds_bytes(const SlidePlan &P) { return lds_bytes(P.slots) + kLdsReduce; }
 
 int slide_pass(mh_ctx *ctx, const SlidePlan &P, const SlideFields &F, const int dims[3],
-               const mh_cmf_params *prm, int lv, int it, bool check, int cur, const SlideControl &C,
-               float *partials, void *inbox, unsigned *tags, hipStream_t s)
+               const mh_cmf_params *prm, int lv, int it, bool check, int cur, bool lost,
+               const SlideControl &C, float *partials, void *inbox, unsigned *tags, hipStream_t s)
 {
     MH_REQUIRE(ctx, lv >= 1 && lv <= P.levels, "levels of a pass");
     const unsigned steps = unsigned(dims[0] + 2 * lv + 4);
@@ -579,7 +579,7 @@ int slide_pass(mh_ctx *ctx, const SlidePlan &P, const SlideFields &F, const int 
     A.slots = P.slots;
     A.levels = lv;
     A.it = it;
-    A.check = check;
+    A.check = int(check) | int(lost) << 1;
     A.cur = cur;
     A.rcc = prm->rcc;
     A.inv_rcc = float(1.0 / double(prm->rcc));

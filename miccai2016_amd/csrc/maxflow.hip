@@ -1363,6 +1363,7 @@ struct Runner {
     // Runner alive (it holds the device's lock until then), taken by choose.
     bool may_slide = false;
     mh::SlidePlan slide;
+    int slid = 0;      // sliding passes launched
     int slide_rc = 0;  // of the last sliding pass: after an error the solve goes on without
     std::unique_lock<std::mutex> slide_lock;
 
@@ -1436,7 +1437,8 @@ struct Runner {
         }
         const mh::SlideControl C{W.ctrl + kStop, W.ctrl + kParity, W.ctrl + kAbort, W.ctrl + kAbortIt,
                                  W.ctrl + kAbortCur};
-        return mh::slide_pass(ctx, slide, F, dims, prm, lv, it, chk, cur, C, W.partials,
+        const bool lost = ctx->lost_group >= 0 && slid >= ctx->lost_group;
+        return mh::slide_pass(ctx, slide, F, dims, prm, lv, it, chk, cur, lost, C, W.partials,
                               ctx->slide_inbox, &ctx->slide_tags, s);
     }
 
@@ -1479,6 +1481,7 @@ struct Runner {
                 ++ctx->chip.refused;
                 return 0;
             }
+            ++slid;
             ++ctx->chip.passes;
             if (chk)
                 hipLaunchKernelGGL(cmf_crit_kernel, dim3(1), dim3(1024), 0, s, W.partials, slide.blocks(),
@@ -1784,6 +1787,7 @@ MH_EXPORT int mh_cmf_solve(mh_ctx *ctx, float *u, const float *eigs, const float
         // input on, which is as it was, the solve takes the other methods
         int at[2];
         MH_CHECK(ctx, hipMemcpy(at, W.ctrl + kAbortIt, sizeof(at), hipMemcpyDeviceToHost));
+        ++ctx->chip.given_up;
         R.may_slide = false;
         R.slide_lock.unlock();
         R.it = at[0];
@@ -3078,13 +3082,22 @@ MH_EXPORT int mh_cmf_set_chip_units(mh_ctx *ctx, int units)
     return MH_OK;
 }
 
-MH_EXPORT int mh_cmf_chip_counts(mh_ctx *ctx, int64_t counts[3])
+MH_EXPORT int mh_cmf_set_lost_group(mh_ctx *ctx, int from)
+{
+    if (!ctx) return MH_ERR_ARG;
+    MH_REQUIRE(ctx, from >= -1, "from >= -1");
+    ctx->lost_group = from;
+    return MH_OK;
+}
+
+MH_EXPORT int mh_cmf_chip_counts(mh_ctx *ctx, int64_t counts[4])
 {
     if (!ctx) return MH_ERR_ARG;
     MH_REQUIRE(ctx, counts, "null pointer");
     counts[0] = ctx->chip.solves;
     counts[1] = ctx->chip.passes;
     counts[2] = ctx->chip.refused;
+    counts[3] = ctx->chip.given_up;
     return MH_OK;
 }
 

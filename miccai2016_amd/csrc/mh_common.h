@@ -59,8 +59,9 @@ struct mh_ctx {
     // compute units that plans of solves on the chip and of sliding passes count
     // on (0: the device's), and what became of them (mh_cmf_chip_counts)
     int chip_units = 0;
+    int lost_group = -1;  // mh_cmf_set_lost_group
     struct {
-        int64_t solves = 0, passes = 0, refused = 0;
+        int64_t solves = 0, passes = 0, refused = 0, given_up = 0;
     } chip;
     // bricks of the on-chip solver per (dims, p-step form, solves)
     std::map<std::array<int, 5>, std::array<int, 6>> onchip_plans;
