@@ -46,10 +46,12 @@ constexpr int kSlideAborted = 3;
 // Enqueue one pass of lv (1 .. plan.levels) iterations from iteration `it`; the
 // device lock must be held until it is done. With `check`, partials[block]
 // receives each work-group's sum of |err| of the last iteration. The tags of
-// the pass follow *tags, which it advances (0: the inbox is new). `lost`: one of
-// its work-groups is missing.
+// the pass follow *tags, which it advances (0: the inbox is new); when they start
+// over, all of the inbox is cleared, the words of larger plans among it. `lost`: one
+// of its work-groups is missing.
 int slide_pass(mh_ctx *ctx, const SlidePlan &plan, const SlideFields &F, const int dims[3],
                const mh_cmf_params *prm, int lv, int it, bool check, int cur, bool lost,
-               const SlideControl &C, float *partials, void *inbox, unsigned *tags, hipStream_t s);
+               const SlideControl &C, float *partials, void *inbox, size_t inbox_bytes, unsigned *tags,
+               hipStream_t s);
 
 }  // namespace mh

@@ -555,12 +555,13 @@ int slide_lds_bytes(const SlidePlan &P) { return lds_bytes(P.slots) + kLdsReduce
 
 int slide_pass(mh_ctx *ctx, const SlidePlan &P, const SlideFields &F, const int dims[3],
                const mh_cmf_params *prm, int lv, int it, bool check, int cur, bool lost,
-               const SlideControl &C, float *partials, void *inbox, unsigned *tags, hipStream_t s)
+               const SlideControl &C, float *partials, void *inbox, size_t inbox_bytes, unsigned *tags,
+               hipStream_t s)
 {
     MH_REQUIRE(ctx, lv >= 1 && lv <= P.levels, "levels of a pass");
     const unsigned steps = unsigned(dims[0] + 2 * lv + 4);
     if (*tags == 0 || *tags > 0xffffffffu - steps) {  // a new inbox, or the tags start over
-        const int64_t words = slide_inbox_bytes(P) / int64_t(sizeof(Word));
+        const int64_t words = int64_t(inbox_bytes / sizeof(Word));
         hipLaunchKernelGGL(zero_words_kernel, dim3(blocks_for(words)), dim3(kBlock), 0, s,
                            static_cast<Word *>(inbox), words);
         MH_CHECK_LAUNCH(ctx, "slide inbox");

@@ -1439,7 +1439,7 @@ struct Runner {
                                  W.ctrl + kAbortCur};
         const bool lost = ctx->lost_group >= 0 && slid >= ctx->lost_group;
         return mh::slide_pass(ctx, slide, F, dims, prm, lv, it, chk, cur, lost, C, W.partials,
-                              ctx->slide_inbox, &ctx->slide_tags, s);
+                              ctx->slide_inbox, ctx->slide_bytes, &ctx->slide_tags, s);
     }
 
     int64_t sweep_grid_of(const SweepMethod &m) const
