@@ -2623,9 +2623,10 @@ MH_EXPORT int mh_cmf_solve_batched(mh_ctx *ctx, float *u, int S, const float *w_
     int first = 0, any_nan = 0;
     // volumes of the sweeps' range: the first pair tunes them for these dims
     // (they run the solves when the device is shared with another on-chip
-    // solve), once per context
-    if (S > 2 && n >= 800000 && prm->num_iter >= 96 &&
-        ctx->sweep_tuned.find({idims[0], idims[1], idims[2]}) == ctx->sweep_tuned.end()) {
+    // solve), once per context, also where its solves stop too early for that
+    if (S > 2 && n >= 800000 && prm->num_iter >= 96 && mh::axi_params(prm).on &&
+        ctx->sweep_tuned.find({idims[0], idims[1], idims[2]}) == ctx->sweep_tuned.end() &&
+        ctx->batch_tried.insert({idims[0], idims[1], idims[2]}).second) {
         const int rc = swept(0, 2);
         if (rc < 0) return rc;
         any_nan |= rc == MH_STOPPED_NAN;

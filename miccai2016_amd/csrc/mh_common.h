@@ -56,6 +56,8 @@ struct mh_ctx {
     // method the batched solver's tuner chose per volume dims (tile shape,
     // plane chunk), timed on pairs of solves
     std::map<std::array<int, 3>, std::pair<int, int>> batch_tuned;
+    // volume dims whose first pair mh_cmf_solve_batched ran to tune the sweeps
+    std::set<std::array<int, 3>> batch_tried;
     // compute units that plans of solves on the chip and of sliding passes count
     // on (0: the device's), and what became of them (mh_cmf_chip_counts)
     int chip_units = 0;
