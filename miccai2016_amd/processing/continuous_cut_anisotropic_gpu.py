@@ -221,7 +221,10 @@ class CmfCutQAnisotropicGpu(TreePrintable):
         P = self._cmf_params((1, 1, 1) if scaling is None else scaling, sq, max(1, u.numel()))
         vd = np.ascontiguousarray(np.asarray(shapes, np.int64).reshape(nv, 3))
         vo = np.ascontiguousarray(np.asarray(offsets, np.int64))
-        work = dev.bytes(_lib.CMF_RAGGED_ONCHIP_BYTES)
+        try:
+            work = dev.bytes(_lib.CMF_RAGGED_ONCHIP_BYTES)
+        except dev.torch.OutOfMemoryError:   # the other solvers may do with less
+            return [None] * nv
         res, solved = (_lib.CmfResult * nv)(), np.zeros(nv, np.int32)
         rc = dev.lib.mh_cmf_ragged_onchip(dev.handle, dev.ptr(u), dev.ptr(quats), dev.ptr(alpha),
                                           dev.ptr(cs), dev.ptr(ct), nv,
