@@ -275,6 +275,11 @@ int mh_gvf(mh_ctx *ctx, float *g3_dev, float *swap3_dev, const float *v3_dev, co
  * depend on it, bit for bit (the magnitude sums of the checks may differ in
  * their summation order). */
 int mh_gvf_set_sweep(mh_ctx *ctx, int mode);
+/* What mode 0 does with a volume on a device of so many compute units (no counterpart
+ * in the reference; host arithmetic only, no context): returns the steps per launch
+ * (1: one) and, where they are more, sets plan (may be NULL) to the voxels of a tile
+ * along axes 1 and 2, its planes along axis 0 and the work-groups of a launch. */
+int mh_gvf_plan(const int64_t dims[3], int iters, int compute_units, int plan[4]);
 
 /* Normalise non-zero vectors of g (SoA x3) to unit length
  * (clcode/gvf.cl:215-232). */

@@ -100,12 +100,11 @@ constexpr int kRawBuffer = 0x00027000;
 // the lanes outside the volume: without branches around them the compiler knows
 // how many are under way and waits for none but the plane it needs. They are
 // issued between the levels (all seven at once hold up the waves at the step's
-// start: 14.3 against 13.2 us per GVF step at 150 x 128 x 141). A step of all
-// work-groups takes about 1.0 + 0.25 L us, the first part for the loads and
-// stores of 64 threads each (tiles of 24 columns 1.2: rows of 128 bytes off
-// their alignment), the second for the arithmetic; so three and four levels in
-// wide tiles win although their halos cost more. Two levels with the loads one
-// plane ahead, which this replaces: 16.7 us; one step per launch: 17.3.
+// start: 8 % more). A step of all work-groups takes about 1.0 + 0.25 L us, the first
+// part for the loads and stores of 64 threads each (tiles of 24 columns 1.2: rows of
+// 128 bytes off their alignment), the second for the arithmetic; so three and four
+// levels often win although their halos cost more: 150 x 128 x 141 11.6 us a GVF step
+// in four levels, 11.7 in three, 13.2 in two (below), 17.0 in one step per launch.
 template <int TY, int TX, int NT, int L>
 __global__ void __launch_bounds__(NT)
 gvf_sweep_kernel(float *__restrict__ out, const float *__restrict__ g, const float *__restrict__ v,
@@ -245,18 +244,157 @@ gvf_sweep_kernel(float *__restrict__ out, const float *__restrict__ g, const flo
     if (t == 0) partials[blockIdx.x] = dsum;
 }
 
+// Two steps per launch in the same way with every plane moved on in registers: 55 of
+// them, so that a compute unit holds two work-groups and one's loads hide behind the
+// other's arithmetic. A plane step of 512 work-groups takes 1.8 us, of 256 1.05; fewer
+// levels read and write more often, so it is the faster while the fields stay in the
+// last-level cache and its tiles fill the device better (128^3 10.7 us a step against
+// 11.3 to 12.8 in three and four levels, 172 x 173 x 122 15.3 and 18.2, 500 x 100 x 60
+// 12.8 and 14.6; but 150 x 128 x 141 13.2 and 11.6, 183 x 158 x 191 22.0 and 20.5).
+template <int TY, int TX, int NT>
+__global__ void __launch_bounds__(NT)
+gvf_two_step_kernel(float *__restrict__ out, const float *__restrict__ g, const float *__restrict__ v,
+                 const float *__restrict__ r, int d0, int d1, int d2, float mu, float dt, float rss0,
+                 float rss1, float rss2, int zchunk, float *__restrict__ partials)
+{
+    constexpr int EY = TY + 4, EX = TX + 4, NE = EY * EX;
+    static_assert(NE <= NT, "one point per thread");
+    __shared__ float sG[2][3][NE];  // g of plane z, by plane parity
+    __shared__ float sH[2][3][NE];  // level-A result of plane z, by plane parity
+    const unsigned b = mh::xcd_block(blockIdx.x, gridDim.x);
+    const int ntx = (d2 + TX - 1) / TX, nty = (d1 + TY - 1) / TY;
+    const int tx = int(b % unsigned(ntx)), ty = int((b / unsigned(ntx)) % unsigned(nty));
+    const int tz = int(b / unsigned(ntx * nty));
+    const int x0 = tx * TX, y0 = ty * TY, z0 = tz * zchunk;
+    const int z1 = min(z0 + zchunk, d0);
+    const int t = int(threadIdx.x);
+    const bool live = t < NE;
+    const int yy = live ? t / EX : 0, xx = live ? t % EX : 0;
+    const int p = yy * EX + xx;
+    const int y = y0 - 2 + yy, x = x0 - 2 + xx;
+    const bool inv = live && y >= 0 && y < d1 && x >= 0 && x < d2;
+    const bool inE1 = inv && yy >= 1 && yy <= TY + 2 && xx >= 1 && xx <= TX + 2;
+    const bool inO = inv && yy >= 2 && yy <= TY + 1 && xx >= 2 && xx <= TX + 1;
+    // in-plane neighbours in LDS, mirrored at the faces (inside E2 for E1)
+    const int pym = y > 0 ? p - EX : p + EX, pyp = y < d1 - 1 ? p + EX : p - EX;
+    const int pxm = x > 0 ? p - 1 : p + 1, pxp = x < d2 - 1 ? p + 1 : p - 1;
+    const int64_t n = int64_t(d0) * d1 * d2, st0 = int64_t(d1) * d2;
+    const int64_t ip = inv ? int64_t(y) * d2 + x : 0;
+    auto at = [&](int z) { return int64_t(z) * st0 + ip; };
+
+    const int zs = max(z0 - 1, 0);  // first level-A plane
+    const int zend = z1;            // last step (level A only below d0)
+    float gm[3], gc[3], gp[3], gn[3];    // g at planes z - 1, z, z + 1 (mirrored), z + 2
+    float vA[3], vB[3], vN[3];           // v at planes z, z - 1, z + 1
+    float rA = 0.f, rB = 0.f, rN = 0.f;
+    float h2[3], h1[3], h0[3];           // level A at planes z - 2, z - 1, z
+    float dsum = 0.f;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        gm[c] = gc[c] = gp[c] = gn[c] = vA[c] = vB[c] = vN[c] = h2[c] = h1[c] = h0[c] = 0.f;
+    }
+    if (inv) {
+        const int zm = zs > 0 ? zs - 1 : zs + 1, zp = zs < d0 - 1 ? zs + 1 : zs - 1;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            gc[c] = g[c * n + at(zs)];
+            gm[c] = g[c * n + at(zm)];
+            gp[c] = g[c * n + at(zp)];
+        }
+    }
+    if (inE1) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) vA[c] = v[c * n + at(zs)];
+        rA = r[at(zs)];
+    }
+    for (int z = zs; z <= zend; ++z) {
+        const bool la = z < d0;                  // level A at plane z
+        const bool lb = z - 1 >= z0;             // level B at plane z - 1 (< z1 since z <= z1)
+        const int q = z & 1, qb = (z - 1) & 1;
+        // inputs of the next step
+        if (inv && z + 1 < d0) {
+            if (z + 2 < d0) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) gn[c] = g[c * n + at(z + 2)];
+            } else {  // plane z + 1 is the last: its upper neighbour mirrors to plane z
+#pragma unroll
+                for (int c = 0; c < 3; ++c) gn[c] = gc[c];
+            }
+        }
+        if (inE1 && z + 1 < d0) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) vN[c] = v[c * n + at(z + 1)];
+            rN = r[at(z + 1)];
+        }
+        if (la && live) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) sG[q][c][p] = gc[c];
+        }
+        __syncthreads();
+        if (la && inE1) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                h0[c] = 0.f;
+                (void)gvf_voxel(gc[c], gm[c], gp[c], sG[q][c][pym], sG[q][c][pyp], sG[q][c][pxm],
+                                sG[q][c][pxp], vA[c], rA, mu, dt, rss0, rss1, rss2, h0[c]);
+                sH[q][c][p] = h0[c];
+            }
+        }
+        if (lb && inO) {
+            const int zb = z - 1;
+            float dl[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const float below = zb > 0 ? h2[c] : h0[c];
+                const float above = zb < d0 - 1 ? h0[c] : h2[c];
+                float o;
+                dl[c] = gvf_voxel(h1[c], below, above, sH[qb][c][pym], sH[qb][c][pyp],
+                                  sH[qb][c][pxm], sH[qb][c][pxp], vB[c], rB, mu, dt, rss0, rss1,
+                                  rss2, o);
+                out[c * n + at(zb)] = o;
+            }
+            if (partials) dsum += gvf_mag(dl[0], dl[1], dl[2]);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            gm[c] = gc[c];
+            gc[c] = gp[c];
+            gp[c] = gn[c];
+            h2[c] = h1[c];
+            h1[c] = h0[c];
+            vB[c] = vA[c];
+            vA[c] = vN[c];
+        }
+        rB = rA;
+        rA = rN;
+    }
+    if (!partials) return;
+    dsum = mh::block_reduce<SumOp>(dsum);
+    if (threadIdx.x == 0) partials[blockIdx.x] = dsum;
+}
+
 struct GvfShape {
     int ty, tx, nt, levels;
-    double unit;  // microseconds a plane step of all resident work-groups takes
+    int per_cu;       // resident work-groups of a compute unit
+    double unit[2];   // microseconds a plane step takes with one and two of them on each
+    int64_t voxels;   // of volumes it is taken for
     const void *kernel;
-    int lds() const { return 4 * levels * 6 * (ty + 2 * levels) * (tx + 2 * levels); }
+    int lds() const { return per_cu > 1 ? 0 : 4 * levels * 6 * (ty + 2 * levels) * (tx + 2 * levels); }
 };
+// (the two-step kernel up to 5.4 million voxels, whose 40 bytes each are 216 MB: at
+// 5.3 and 5.1 million it is the faster by 5 and 13 % where it is chosen, at 5.5 and 5.8
+// million the slower by 7 and 9 %)
 #define GVF_SHAPE(TY, TX, NT, L, UNIT) \
-    {TY, TX, NT, L, UNIT, reinterpret_cast<const void *>(&gvf_sweep_kernel<TY, TX, NT, L>)}
-const GvfShape kGvfShapes[] = {GVF_SHAPE(15, 48, 1024, 2, 1.6), GVF_SHAPE(12, 50, 1024, 3, 1.6),
+    {TY, TX, NT, L, 1, {UNIT, UNIT}, int64_t(1) << 31, \
+     reinterpret_cast<const void *>(&gvf_sweep_kernel<TY, TX, NT, L>)}
+#define GVF_PAIR(TY, TX) \
+    {TY, TX, 1024, 2, 2, {1.45, 2.55}, 5400000, \
+     reinterpret_cast<const void *>(&gvf_two_step_kernel<TY, TX, 1024>)}
+const GvfShape kGvfShapes[] = {GVF_PAIR(11, 64), GVF_PAIR(12, 60), GVF_SHAPE(12, 50, 1024, 3, 1.6),
                                GVF_SHAPE(10, 58, 1024, 3, 1.52), GVF_SHAPE(6, 74, 960, 3, 1.34),
                                GVF_SHAPE(24, 24, 1024, 4, 1.95)};
 #undef GVF_SHAPE
+#undef GVF_PAIR
 
 // Sum of the per-block partials in block order (one work-group).
 __global__ void __launch_bounds__(mh::kBlock)
@@ -315,34 +453,38 @@ struct GvfPlan {
     int64_t groups = 0;
 };
 
-// The shape and plane chunk that take the fewest microseconds per step: a
-// launch's work-groups run in ceil(groups / slots) waves of chunk + 2 (levels - 1)
-// plane steps, and a launch costs 2.5 beside them; the chunk must leave at most
-// max_groups groups. One step per launch takes 2.2 + 5.6 per million voxels, the
-// less up to about 80^3 (5.2 us a step there, 5.5 in three levels; 96^3 7.2 and
-// 5.8, 120^3 11.9 and 8.7, 220 x 215 x 210 94 and 41). `any`: a sweep in any case.
-GvfPlan gvf_plan(mh_ctx *ctx, const int64_t dims[3], int iters, int64_t max_groups, bool any)
+// The shape and plane chunk that take the fewest microseconds per step on a device
+// of `cus` compute units: a launch's work-groups run in ceil(groups / resident ones)
+// waves of chunk + 2 (levels - 1) plane steps, and a launch costs 2.5 beside them; the
+// chunk must leave at most max_groups groups. One step per launch takes 2.2 + 5.6 per
+// million voxels, the less up to about 80^3 (4.9 us a step there, 5.2 in three levels;
+// 96^3 6.6 and 5.4, 110^3 9.6 and 6.6, 220 x 215 x 210 93 and 38). `any`: a sweep in
+// any case. (Of 95 volumes of 0.15 to 33 million voxels the plan's choice is on
+// average 1.0 % off the fastest shape and chunk, at most 13 %.)
+GvfPlan gvf_plan(int cus, const int64_t dims[3], int iters, int64_t max_groups, bool any)
 {
     GvfPlan best;
-    if (4 * dims[1] * dims[2] >= (int64_t(1) << 31)) return best;  // bytes of a buffer resource
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
-        cus <= 0)
-        cus = 256;
-    double cost = any ? 1e30 : 2.2 + 5.6e-6 * double(dims[0]) * double(dims[1]) * double(dims[2]);
+    // planes beyond the bytes of a buffer resource: the two-step kernel has none (and
+    // volumes of such planes read the less from memory)
+    const bool wide = 4 * dims[1] * dims[2] >= (int64_t(1) << 31);
+    double cost = any || wide ? 1e30 : 2.2 + 5.6e-6 * double(dims[0]) * double(dims[1]) * double(dims[2]);
     if (cost < 3.0) return best;  // no sweep takes less
     const int d0 = int(dims[0]);
     for (const GvfShape &S : kGvfShapes) {
         if (iters < S.levels) continue;
+        if (wide ? S.per_cu == 1 : !any && dims[0] * dims[1] * dims[2] > S.voxels) continue;
         const int64_t tiles = ((dims[2] + S.tx - 1) / S.tx) * ((dims[1] + S.ty - 1) / S.ty);
+        const int64_t slots = int64_t(cus) * S.per_cu;
         // as many chunks as fill the device once, twice, ..
         for (int64_t waves = (tiles + cus - 1) / cus, k = 0; k < 8; ++waves, ++k) {
             const int chunks = int(std::min<int64_t>(d0, waves * cus / tiles));
             const int z = (d0 + chunks - 1) / chunks;
             const int64_t groups = tiles * ((d0 + z - 1) / z);
             if (groups > max_groups) break;
-            const double c = (double((groups + cus - 1) / cus) * (z + 2 * (S.levels - 1)) * S.unit + 2.5) /
-                             S.levels;
+            const int64_t rest = groups % slots;
+            const double step = double(groups / slots) * S.unit[S.per_cu - 1] +
+                                (rest == 0 ? 0.0 : S.unit[rest <= cus ? 0 : 1]);
+            const double c = ((z + 2 * (S.levels - 1)) * step + 2.5) / S.levels;
             if (c < cost) {
                 cost = c;
                 best.shape = &S;
@@ -351,8 +493,30 @@ GvfPlan gvf_plan(mh_ctx *ctx, const int64_t dims[3], int iters, int64_t max_grou
             }
         }
     }
-    (void)hipGetLastError();
     return best;
+}
+
+int gvf_compute_units(mh_ctx *ctx)
+{
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess ||
+        cus <= 0)
+        cus = 256;
+    (void)hipGetLastError();
+    return cus;
+}
+
+MH_EXPORT int mh_gvf_plan(const int64_t dims[3], int iters, int compute_units, int plan[4])
+{
+    if (!mh::dims_ok(dims) || compute_units < 1) return MH_ERR_ARG;
+    const GvfPlan P = gvf_plan(compute_units, dims, iters,
+                               int64_t(mh::blocks_for(dims[0] * dims[1] * dims[2])), false);
+    if (!P.shape) return 1;
+    if (plan) {
+        const int v[4] = {P.shape->ty, P.shape->tx, P.zchunk, int(P.groups)};
+        std::copy(v, v + 4, plan);
+    }
+    return P.shape->levels;
 }
 
 MH_EXPORT int mh_gvf(mh_ctx *ctx, float *g3, float *swap3, const float *v3, const float *r,
@@ -371,7 +535,7 @@ MH_EXPORT int mh_gvf(mh_ctx *ctx, float *g3, float *swap3, const float *v3, cons
     // last launch fit in the workspace's nb floats
     GvfPlan P;
     if (ctx->gvf_sweep != 1 && iters >= 2)
-        P = gvf_plan(ctx, dims, iters, int64_t(nb), ctx->gvf_sweep == 2);
+        P = gvf_plan(gvf_compute_units(ctx), dims, iters, int64_t(nb), ctx->gvf_sweep == 2);
     const int levels = P.shape ? P.shape->levels : 1;
     if (P.shape)
         MH_CHECK(ctx, hipFuncSetAttribute(P.shape->kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
