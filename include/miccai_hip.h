@@ -330,9 +330,9 @@ int mh_cmf_solve(mh_ctx *ctx, float *u_dev, const float *eigs_dev, const float *
  * process ends, so volumes are limited to MH_CMF_NOALLOC_MAX_VOXELS voxels
  * (larger ones are rejected with MH_ERR_ARG). Same arguments, results (bit
  * for bit) and blocking as mh_cmf_solve; the context's device must be
- * current. The method is the one mh_cmf_solve tuned for these dims on this
- * context, else the untuned default; it never tunes and never captures a
- * graph. Every call on a GPU shares its array: calls that overlap on one GPU
+ * current. What fits stays on the chip as in mh_cmf_solve; otherwise the method
+ * is the one mh_cmf_solve tuned for these dims on this context, else the untuned
+ * default; it never tunes, takes no sliding passes and never captures a graph. Every call on a GPU shares its array: calls that overlap on one GPU
  * (other streams or threads) race and must be serialised by the caller. */
 #define MH_CMF_NOALLOC_MAX_VOXELS (1 << 20)
 int mh_cmf_solve_noalloc(mh_ctx *ctx, float *u_dev, const float *eigs_dev, const float *alpha_dev,
@@ -417,9 +417,9 @@ int mh_cmf_set_chip_units(mh_ctx *ctx, int units);
  * what another sends (another process on the same device may keep that from running);
  * then the launch ends, its solves are as before it and take other methods. */
 int mh_cmf_chip_counts(mh_ctx *ctx, int64_t counts[4]);
-/* For tests of that: from solve `from` of a launch on the chip, and from sliding pass
- * `from` of a solve, one work-group is missing (-1, the default: none is). Results do
- * not depend on it, bit for bit. */
+/* For tests of that: from sliding pass `from` of a solve on, and (0) in every launch on
+ * the chip, the last of the work-groups is missing if there are several (-1, the
+ * default: none is). Results do not depend on it, bit for bit. */
 int mh_cmf_set_lost_group(mh_ctx *ctx, int from);
 /* Graph replay in mh_cmf_solve and the resident solves (no counterpart in the
  * reference): when the per-iteration kernels run, one criterion cycle (update

@@ -68,7 +68,6 @@ constexpr int kPointwise = 2;  // eigenvalues of their own at every voxel
 struct Args {
     const mh::OnchipSolve *solves;
     int nsolves, nslots;
-    int nfirst;  // solves the first brick takes part in: all (mh_cmf_set_lost_group: fewer)
     mh::OnchipFields F;
     int d0, d1, d2;
     int b1, b2, nt1, nt2, nz;
@@ -188,8 +187,7 @@ cmf_onchip_kernel(const ArgsOf<N> L)
 
     // Receives this thread's words: one load of each as its phase ends, then
     // all of them again until none is missing. (The first load half a phase
-    // earlier mostly came too early: 5.6 against 4.9 us per iteration at
-    // 128^3.) The axis-0 neighbour's value is returned, the in-plane ones go to
+    // earlier mostly came too early: 14 % slower at 128^3.) The axis-0 neighbour's value is returned, the in-plane ones go to
     // `tile`.
     Word first[R + 1];
     auto look = [&](unsigned zoff, bool rz, unsigned off, const bool (&rv)[R]) {
@@ -244,8 +242,7 @@ cmf_onchip_kernel(const ArgsOf<N> L)
 
     unsigned tag = 1;
     int nparts = 0;
-    const int nsolves = lb == 0 ? A.nfirst : A.nsolves;
-    for (int q = slot; q < nsolves; q += A.nslots) {
+    for (int q = slot; q < A.nsolves; q += A.nslots) {
         float h0[V], h1[V], h2[V], pt[V], u[V], al[V], cs[V], ct[V], fr[V][NF];
         unsigned lab = 0;
         {
@@ -551,8 +548,9 @@ const void *kernel_sup(bool sup)
 
 // The kernel of a brick of v planes. The criterion is settled during the next
 // iteration's p-step, except where that costs registers that are not there and
-// a criterion is rare (8 planes, 128^3: 4.7 us per iteration with a criterion
-// every 30 against 5.0 in the p-step; 8.7 against 5.9 with one every iteration).
+// a criterion is rare (8 planes, 128^3: 4.6 us per iteration with a criterion
+// every 30, 6 % more in the p-step; with one every iteration 6.0 in the p-step, 47 %
+// more out of it).
 const void *kernel_of(int v, int mode, bool sup, int update)
 {
     const bool rare = update >= 8;
@@ -579,10 +577,11 @@ bool plan_fits(const mh::OnchipPlan &P)
     return nc <= kMaxThreads && words_of(P) <= kWords * threads_of(P) && nc + P.b1 + P.b2 + 1 <= kCells;
 }
 
-// Microseconds of an iteration, from measured plans (8 planes of 8 x 128
-// voxels per brick 4.9, of 8 x 64 3.4; 4 of 10 x 96 3.7, of 8 x 64 2.6; 2 of
-// 8 x 64 2.6; 1 of 10 x 37 2.3, of 16 x 64 3.4; bricks split along axis 2: 8 of
-// 16 x 64 6.3, 4 of 32 x 32 4.8): the two exchanges, the issue of a SIMD's waves
+// Microseconds of an iteration, fitted to plans as an earlier, up to 7 % slower form
+// of the kernel ran them (8 planes of 8 x 128 voxels per brick 4.9, now 4.6; of 8 x 64
+// 3.4; 4 of 10 x 96 3.7, of 8 x 64 2.6; 2 of 8 x 64 2.6; 1 of 10 x 37 2.3, of 16 x 64
+// 3.4; bricks split along axis 2: 8 of 16 x 64 6.3, 4 of 32 x 32 4.8), whose order is
+// what the choice goes by: the two exchanges, the issue of a SIMD's waves
 // plane by plane (one wave alone does not hide its own latencies), the axis-0
 // words where little work covers them, and along a split axis 2 the words every
 // wave sends last.
@@ -662,9 +661,10 @@ int64_t nwords_of(const OnchipPlan &P, int slots)
 {
     return int64_t(slots) * P.blocks() * (2 * (P.b1 * P.b2 + words_of(P)) + 2);
 }
-int first_brick_solves(mh_ctx *ctx, int solves)
+// work-groups launched of so many: all, but for mh_cmf_set_lost_group
+unsigned launched(mh_ctx *ctx, int blocks)
 {
-    return ctx->lost_group < 0 ? solves : std::min(ctx->lost_group, solves);
+    return unsigned(ctx->lost_group == 0 ? std::max(1, blocks - 1) : blocks);
 }
 Args args_of(const OnchipPlan &P, const OnchipFields &F, const int dims[3], const mh_cmf_params *prm)
 {
@@ -769,7 +769,6 @@ int onchip_run_many(mh_ctx *ctx, const OnchipVolume *vols, int nvol, const mh_cm
         A.abort = abort;
         A.solves = table + v;
         A.nsolves = A.nslots = 1;
-        A.nfirst = first_brick_solves(ctx, 1);
         Few few{};
         few.s[0] = V.solve;
         hipLaunchKernelGGL(onchip_prepare_kernel,
@@ -783,7 +782,7 @@ int onchip_run_many(mh_ctx *ctx, const OnchipVolume *vols, int nvol, const mh_cm
     const int lds = lds_bytes(8, kAxial);
     void *args[] = {&L};
     MH_CHECK(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(unsigned(L.first[nvol])),
+    const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(launched(ctx, L.first[nvol])),
                                                     dim3(unsigned(threads)), args, unsigned(lds), s);
     if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -858,7 +857,6 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     A.solves = table;
     A.nsolves = nsolves;
     A.nslots = slots;
-    A.nfirst = first_brick_solves(ctx, nsolves);
     Few few{};
     if (nsolves <= kFew)
         std::copy(solves, solves + nsolves, few.s);
@@ -871,7 +869,7 @@ int onchip_run(mh_ctx *ctx, const OnchipPlan &P, const OnchipSolve *solves, int 
     MH_CHECK_LAUNCH(ctx, "onchip prepare");
     void *args[] = {&L};
     MH_CHECK(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-    const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(unsigned(slots * P.blocks())),
+    const hipError_t e = hipLaunchCooperativeKernel(kernel, dim3(launched(ctx, slots * P.blocks())),
                                                     dim3(unsigned(threads_of(P))), args,
                                                     unsigned(lds), s);
     if (e != hipSuccess) {  // the device does not hold every work-group: nothing ran

@@ -9,7 +9,7 @@
 // plane s is new and plane s - 2 levels leaves. A pass of L levels over D0 planes
 // takes D0 + 2 L steps, reads and writes the state once, and recomputes
 // nothing: the in-plane faces of neighbouring tiles and the axis-0 faces between
-// runs of planes travel as tagged words (cmf_words.h).
+// runs of planes (one run's with itself) travel as tagged words (cmf_words.h).
 //
 // Step s, all planes of parity s:
 //   barrier; p-step: residuals of the plane and the next one (LDS; the run's
@@ -80,7 +80,7 @@ struct Args {
     SlideControl C;
     int d0, d1, d2;
     int b1, b2, nt1, nt2, slots;
-    int levels, it, check, cur;  // check & 2: the last work-group is missing
+    int levels, it, check, cur;
     float rcc, inv_rcc, rs0, rs1, rs2, ss0, ss1, ss2;
     AxiParams A;
     Word *inbox;  // per work-group: [axis-0 residuals | h0 | rows and columns of residuals | of h]
@@ -108,11 +108,13 @@ __device__ __forceinline__ const Vec<2> &half(const Vec<4> *p, int h)
     return reinterpret_cast<const Vec<2> *>(p)[h];
 }
 
-template <bool SUP>
+// ONE: one run per tile (an instance of its own: the wrapped positions cost the others
+// 1 %)
+template <bool SUP, bool ONE>
 __global__ void __launch_bounds__(kMaxThreads)
 cmf_slide_kernel(const Args A)
 {
-    if (*A.C.stop || ((A.check & 2) && blockIdx.x > 0 && blockIdx.x == gridDim.x - 1)) return;
+    if (*A.C.stop) return;
     using Vec4 = Vec<4>;
     using Vec2 = Vec<2>;
     extern __shared__ __align__(16) unsigned char lds[];
@@ -316,10 +318,10 @@ cmf_slide_kernel(const Args A)
             over0 = (unsigned(__ballot(k > 0)) & 1u) != 0;
         }
         const unsigned act = adv & kMine, out = mask >> 8 & kMine;
-        // planes s, s - 1 and s - 2 levels: their positions, from 0 to W - 1 (of this
-        // run's if below kRun; with one run per tile, W = kRun, all of them are)
-        const int joins = s < A.d0 ? (ph >= 1 ? ph - 1 : W - 1) : -1;
-        const int settles = s <= A.d0 && s > 0 ? (ph >= 2 ? ph - 2 : ph - 2 + W) : -1;
+        // positions of planes s, s - 1 and s - 2 levels, this run's if 0 .. kRun - 1 (-1
+        // and -2 are W - 1 and W - 2, another run's but where the tile has one run)
+        const int joins = s < A.d0 ? (ONE && ph < 1 ? W - 1 : ph - 1) : -1;
+        const int settles = s <= A.d0 && s > 0 ? (ONE && ph < 2 ? ph - 2 + W : ph - 2) : -1;
         const int leaves = s >= lv2 ? (ph - 1 < lv2 ? ph - 1 - lv2 + W : ph - 1 - lv2) : -1;
         lds_barrier();
         Vec4 *own = own_cell(t8);
@@ -470,7 +472,7 @@ cmf_slide_kernel(const Args A)
         *A.C.stop = kSlideAborted;
         return;
     }
-    if (A.check & 1) A.partials[b] = aerr;
+    if (A.check) A.partials[b] = aerr;
     if (b == 0) *A.C.parity = 1 - A.cur;
 }
 
@@ -478,6 +480,13 @@ __global__ void __launch_bounds__(mh::kBlock) zero_words_kernel(Word *w, int64_t
 {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i < n) w[i] = 0;
+}
+
+template <bool ONE>
+const void *kernel_of(bool sup)
+{
+    return sup ? reinterpret_cast<const void *>(&cmf_slide_kernel<true, ONE>)
+               : reinterpret_cast<const void *>(&cmf_slide_kernel<false, ONE>);
 }
 
 int threads_of(const SlidePlan &P) { return (P.b1 * P.b2 + 63) / 64 * 64; }
@@ -539,8 +548,9 @@ SlidePlan slide_plan(int cus, const int dims[3], const mh_cmf_params *prm, bool 
     // against 2.18e11 here, 192^3 1.28e11 and 1.49e11, 240 x 230 x 190 1.17e11 and
     // 1.63e11, 320^3 1.2e11 and 1.36e11; but 420^3 1.30e11 and 0.92e11, 256^3 with a
     // criterion every 5 iterations 1.1e11 and 0.82e11), and with seeds against the
-    // per-iteration kernels (256^3 5.6e10 and 2.08e11, 128 x 512 x 512 5.7e10 and
-    // 1.2e11).
+    // per-iteration kernels (256^3 5.6e10 and 2.08e11; with one run of planes, three
+    // iterations a pass, 128 x 512 x 512 5.7e10 and 1.14e11, 40 x 512 x 512 6.0e10 and
+    // 1.02e11, 64 x 400 x 400 6.0e10 and 7.9e10, 10 x 500 x 500 6.3e10 and 6.8e10).
     const double others = sup ? 6e4 : n < (int64_t(1) << 22) ? 1.5e5 : 1.3e5;
     if (best.levels && best_cost > double(n) / others) best.levels = 0;
     return best;
@@ -580,7 +590,7 @@ int slide_pass(mh_ctx *ctx, const SlidePlan &P, const SlideFields &F, const int 
     A.slots = P.slots;
     A.levels = lv;
     A.it = it;
-    A.check = int(check) | int(lost) << 1;
+    A.check = check;
     A.cur = cur;
     A.rcc = prm->rcc;
     A.inv_rcc = float(1.0 / double(prm->rcc));
@@ -595,11 +605,11 @@ int slide_pass(mh_ctx *ctx, const SlidePlan &P, const SlideFields &F, const int 
     A.tag0 = *tags;
     A.partials = partials;
     *tags += steps;
-    const void *kernel = F.labels ? reinterpret_cast<const void *>(&cmf_slide_kernel<true>)
-                                  : reinterpret_cast<const void *>(&cmf_slide_kernel<false>);
+    const void *kernel = P.slots == 1 ? kernel_of<true>(F.labels != nullptr) : kernel_of<false>(F.labels != nullptr);
     void *args[] = {&A};
     MH_CHECK(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(P.slots)));
-    MH_CHECK(ctx, hipLaunchCooperativeKernel(kernel, dim3(unsigned(P.blocks())),
+    const unsigned blocks = unsigned(P.blocks() - (lost && P.blocks() > 1));
+    MH_CHECK(ctx, hipLaunchCooperativeKernel(kernel, dim3(blocks),
                                              dim3(unsigned(threads_of(P))), args,
                                              unsigned(lds_bytes(P.slots)), s));
     return MH_OK;

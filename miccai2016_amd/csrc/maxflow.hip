@@ -1717,8 +1717,8 @@ int solve_core(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, con
 }
 
 // The solve with its whole state on the chip, where the context's settings
-// leave the method open and the volume fits (the 128^3 cell: 2.7 times the
-// tuned sweep; the smallest volumes: twice the per-iteration kernels). Waits
+// leave the method open and the volume fits (the 128^3 cell: 3.4 times the
+// tuned sweep; the smallest volumes: twice the per-iteration kernels and more). Waits
 // for it; `ran` false: u is unchanged and nothing was done.
 int solve_onchip(mh_ctx *ctx, float *u, const float *eigs, const float *alpha, const float *cs,
                  const float *ct, const uint8_t *labels, const Dims D, int64_t n,
