@@ -656,6 +656,7 @@ OnchipPlan onchip_plan(mh_ctx *ctx, const int dims[3], const mh_cmf_params *prm,
             }
         }
     }
+    if (ctx->onchip_plans.size() >= 4096) ctx->onchip_plans.clear();  // (formed again in microseconds)
     ctx->onchip_plans[key] = {best.v, best.b1, best.b2, best.nt1, best.nt2, best.nz};
     return best;
 }
